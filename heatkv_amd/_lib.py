@@ -71,6 +71,13 @@ SIGNATURES = {
          _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, ctypes.c_float, _c_i32, _c_i32,
          _c_i32, _c_p, _c_i32, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_p],
     ),
+    "hkv_segmented_attention_split_bytes": (_c_i64, [_c_i32, _c_i32, _c_i32, _c_i64, _c_i32]),
+    "hkv_segmented_attention_split": (
+        _c_i32,
+        [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i32, _c_i32, _c_i32,
+         _c_i64, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, ctypes.c_float, _c_i32, _c_i32,
+         _c_i32, _c_p, _c_i32, _c_p, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p],
+    ),
     "hkv_segmented_attention_noalloc": (
         _c_i32,
         [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i32, _c_i32, _c_i32,

@@ -364,6 +364,91 @@ int32_t hkv_segmented_attention_append2(const void* q, void* slab_k, void* slab_
   return ok();
 }
 
+int64_t hkv_segmented_attention_split_bytes(int32_t batch, int32_t heads, int32_t cur_len, int64_t slab_capacity,
+                                            int32_t v_dtype) {
+  if (batch <= 0 || heads <= 0 || cur_len <= 0 || slab_capacity < 0 || elem_bytes(v_dtype) == 0)
+    return fail(HKV_ERR_INVALID_ARG, "batch, heads and cur_len must be positive, slab_capacity >= 0, v_dtype known");
+  ok();
+  const int64_t rows = static_cast<int64_t>(batch) * (slab_capacity + static_cast<int64_t>(heads) * cur_len);
+  return rows * 512 * (v_dtype == HKV_DTYPE_F32 ? 2 : 1);
+}
+
+int32_t hkv_segmented_attention_split(const void* q, void* slab_k, void* slab_v, const int32_t* seg_starts,
+                                      const int32_t* seg_ends, const int32_t* seg_counts, const void* cur_k,
+                                      const void* cur_v, void* out, float* lse, int32_t batch, int32_t heads,
+                                      int32_t cur_len, int64_t slab_capacity, int32_t max_segments,
+                                      int32_t head_dim, int32_t q_dtype, int32_t k_dtype, int32_t v_dtype,
+                                      int32_t out_dtype, float softmax_scale, int32_t use_exp2, int32_t qk_dot_mode,
+                                      int32_t value_dot_mode, const int32_t* work_plan, int32_t plan_units,
+                                      void* workspace, int64_t workspace_bytes, const int32_t* append_offsets,
+                                      void* slab2_k, void* slab2_v, int64_t slab2_capacity,
+                                      const int32_t* append2_offsets, void* scratch, int64_t scratch_bytes,
+                                      void* stream) {
+  hkv::AttnArgs a{};
+  const int32_t code = build_attention_args(
+      a, true, q, slab_k, slab_v, seg_starts, seg_ends, seg_counts, cur_k, cur_v, out, lse, batch, heads, cur_len,
+      slab_capacity, max_segments, head_dim, q_dtype, k_dtype, v_dtype, out_dtype, softmax_scale, use_exp2,
+      qk_dot_mode, value_dot_mode, work_plan, plan_units, workspace, workspace_bytes, append_offsets, slab2_k,
+      slab2_v, slab2_capacity, append2_offsets);
+  if (code != 0) return code;
+  const bool with_v = v_dtype == HKV_DTYPE_F32;
+  if (q_dtype != HKV_DTYPE_F32 || k_dtype != HKV_DTYPE_F32 || qk_dot_mode == 2 || value_dot_mode == 2)
+    return fail(HKV_ERR_UNSUPPORTED,
+                "the split call takes float32 q and k and the default (or tf32) dot modes (got q %d, k %d, modes "
+                "%d/%d)", q_dtype, k_dtype, qk_dot_mode, value_dot_mode);
+  // the split reads its rows 16 bytes per access
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(slab_k) | reinterpret_cast<uintptr_t>(cur_k) |
+                         (with_v ? reinterpret_cast<uintptr_t>(slab_v) | reinterpret_cast<uintptr_t>(cur_v) : 0) |
+                         reinterpret_cast<uintptr_t>(scratch);
+  if ((bits & 15) != 0) return fail(HKV_ERR_INVALID_ARG, "the split needs 16-byte aligned fp32 tensors and scratch");
+  const int64_t need = hkv_segmented_attention_split_bytes(batch, heads, cur_len, slab_capacity, v_dtype);
+  if (!scratch || scratch_bytes < need)
+    return fail(HKV_ERR_INVALID_ARG, "scratch of %lld bytes is smaller than the %lld required",
+                static_cast<long long>(scratch ? scratch_bytes : 0), static_cast<long long>(need));
+  const int64_t slab_bytes = static_cast<int64_t>(batch) * slab_capacity * 512;
+  const int64_t cur_rows = static_cast<int64_t>(batch) * heads * cur_len;
+  uint8_t* const s = static_cast<uint8_t*>(scratch);
+  hkv::SplitOperands o{};
+  o.slab_k = static_cast<const float*>(slab_k);
+  o.cur_k = static_cast<const float*>(cur_k);
+  o.cur_k_out = s;
+  o.slab_k_out = s + cur_rows * 512;
+  if (with_v) {
+    o.slab_v = static_cast<const float*>(slab_v);
+    o.cur_v = static_cast<const float*>(cur_v);
+    o.cur_v_out = o.slab_k_out + slab_bytes;
+    o.slab_v_out = o.cur_v_out + cur_rows * 512;
+  }
+  o.seg_starts = seg_starts;
+  o.seg_ends = seg_ends;
+  o.seg_counts = seg_counts;
+  o.slab_capacity = slab_capacity;
+  o.cur_rows = cur_rows;
+  o.batch = batch;
+  o.heads = heads;
+  o.max_segments = max_segments;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  hipError_t e = hkv::launch_split_operands(o, with_v, st);
+  if (e == hipSuccess) {
+    hkv::AttnArgs b = a;
+    b.slab_k = o.slab_k_out;
+    b.cur_k = o.cur_k_out;
+    b.k_dtype = hkv::kSplitRows;
+    if (with_v) {
+      b.slab_v = o.slab_v_out;
+      b.cur_v = o.cur_v_out;
+      b.v_dtype = hkv::kSplitRows;
+    }
+    b.append_offsets = nullptr;
+    b.append2_offsets = nullptr;
+    e = hkv::launch_segmented_attention(b, st);
+  }
+  if (e == hipSuccess && append_offsets != nullptr) e = hkv::launch_append(a, st);
+  if (e != hipSuccess)
+    return fail(HKV_ERR_LAUNCH, "segmented attention launch failed: %s", hipGetErrorString(e));
+  return ok();
+}
+
 // The argument block of hkv_segmented_attention_bind: the validated launch
 // arguments, the device they were validated for and a tag.
 namespace {

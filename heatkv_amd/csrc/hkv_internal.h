@@ -116,6 +116,33 @@ int32_t attention_item_queries(const AttnArgs& a);
 int32_t attention_workgroups_per_cu(const AttnArgs& a);
 hipError_t launch_split_rows(const float* src, void* dst, int64_t rows, hipStream_t stream);
 
+// fp32 operands of one attention call to split rows in one launch: the current
+// rows [cur_rows, 128] of K and V, and the slab rows that the tables hold
+// (written at the same row of the *_out slab; the other rows stay unwritten).
+struct SplitOperands {
+  const float* slab_k;
+  const float* slab_v;
+  const float* cur_k;
+  const float* cur_v;
+  uint8_t* slab_k_out;
+  uint8_t* slab_v_out;
+  uint8_t* cur_k_out;
+  uint8_t* cur_v_out;
+  const int32_t* seg_starts;
+  const int32_t* seg_ends;
+  const int32_t* seg_counts;
+  int64_t slab_capacity;
+  int64_t cur_rows;     // batch * heads * cur_len
+  int64_t slab_blocks;  // set by the launch
+  int32_t batch;
+  int32_t heads;
+  int32_t max_segments;
+  int32_t slab_chunks;  // set by the launch
+};
+hipError_t launch_split_operands(SplitOperands o, bool with_v, hipStream_t stream);
+// The append of AttnArgs::append_offsets as a launch of its own.
+hipError_t launch_append(const AttnArgs& a, hipStream_t stream);
+
 constexpr int kMaxSegments = 256;
 
 // Round split of the 16-bit attention kernel (workspace layout): kCounterBytes

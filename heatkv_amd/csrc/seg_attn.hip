@@ -16,6 +16,15 @@ __global__ __launch_bounds__(256) void append_kernel(const AttnArgs a, int32_t k
   attn::append_block<256>(a, blockIdx.x, k_row, v_row);
 }
 
+bool force_staged() {
+  static const bool v = [] {
+    const char* e = std::getenv("HKV_ATTN_PATH");
+    return e != nullptr && std::strcmp(e, "staged") == 0;
+  }();
+  return v;
+}
+}  // namespace
+
 hipError_t launch_append(const AttnArgs& a, hipStream_t stream) {
   const int64_t blocks = attn::append_blocks(a.batch, a.heads, a.cur_len);
   if (blocks <= 0) return hipSuccess;
@@ -26,15 +35,6 @@ hipError_t launch_append(const AttnArgs& a, hipStream_t stream) {
   append_kernel<<<dim3(static_cast<uint32_t>(blocks)), 256, 0, stream>>>(a, k_row, v_row);
   return hipGetLastError();
 }
-
-bool force_staged() {
-  static const bool v = [] {
-    const char* e = std::getenv("HKV_ATTN_PATH");
-    return e != nullptr && std::strcmp(e, "staged") == 0;
-  }();
-  return v;
-}
-}  // namespace
 
 int32_t attention_workgroups_per_cu(const AttnArgs& a) {
   if (a.k_dtype == kSplitRows) return 1;

@@ -1,5 +1,5 @@
-// Segmented attention for fp32 q and k with 16-bit V at the default dot modes:
-// split-bf16 products fed by DMA, software-pipelined.
+// Segmented attention for fp32 q and k at the default dot modes (16-bit V, or
+// fp32 V split like K): split-bf16 products fed by DMA, software-pipelined.
 //
 // K arrives as split rows (dtype code kSplitRows): each row of 128 fp32
 // values is stored as its 128 bf16 high parts, then its 128 bf16 low parts
@@ -136,6 +136,85 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
   uint8_t* const out = dst + row * kSRowBytes;
   *reinterpret_cast<u32x4_t*>(out + c * 16) = hi;
   *reinterpret_cast<u32x4_t*>(out + kD * 2 + c * 16) = lo;
+}
+
+// What an attention call on fp32 K (and V) rows splits before it: the current
+// rows, and of the slab only the rows that the tables' segments hold, K and V
+// (blockIdx.y) in one launch.  A block moves 64 rows at a time, 16 threads per
+// row, 4 rows' loads in flight per thread.  A head's retained rows are one
+// stream (its segments back to back) that slab_chunks blocks share, and the
+// slab's blocks come first: they wait for the tables, and one long head must
+// not end the launch late (2304 tokens, 16 heads, B = 2, K and V, 75 MB in and
+// 75 MB out: 34 us, against 110 us with one block per head).
+constexpr int kSplitBlockRows = 64;
+constexpr int64_t kSplitSlabBlocks = 512;  // about as many for the slab: most find few rows or none
+
+__device__ __forceinline__ void split_row_group(const float* src, uint8_t* dst, const int64_t (&rows)[4]) {
+  const int c = threadIdx.x & 15;
+  f32x4_t x[4], y[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    if (rows[u] < 0) continue;
+    x[u] = *reinterpret_cast<const f32x4_t*>(src + rows[u] * kD + c * 8);
+    y[u] = *reinterpret_cast<const f32x4_t*>(src + rows[u] * kD + c * 8 + 4);
+  }
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    if (rows[u] < 0) continue;
+    const float v[8] = {x[u][0], x[u][1], x[u][2], x[u][3], y[u][0], y[u][1], y[u][2], y[u][3]};
+    u32x4_t hi, lo;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      hi[k] = pack2<kBF16>(v[2 * k], v[2 * k + 1]);
+      const float h0 = __builtin_bit_cast(float, hi[k] << 16);
+      const float h1 = __builtin_bit_cast(float, hi[k] & 0xffff0000u);
+      lo[k] = pack2<kBF16>(v[2 * k] - h0, v[2 * k + 1] - h1);
+    }
+    uint8_t* const out = dst + rows[u] * kSRowBytes;
+    *reinterpret_cast<u32x4_t*>(out + c * 16) = hi;
+    *reinterpret_cast<u32x4_t*>(out + kD * 2 + c * 16) = lo;
+  }
+}
+
+__global__ __launch_bounds__(256) void split_operands_kernel(const SplitOperands o) {
+  __shared__ int32_t seg_start[kMaxSegments];
+  __shared__ int32_t seg_pref[kMaxSegments + 1];
+  const bool is_v = blockIdx.y != 0;
+  const int sub = threadIdx.x >> 4;
+  const int64_t blk = blockIdx.x;
+  int64_t rows[4];
+  if (blk >= o.slab_blocks) {
+    const int64_t r0 = (blk - o.slab_blocks) * kSplitBlockRows;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t r = r0 + sub + 16 * u;
+      rows[u] = r < o.cur_rows ? r : -1;
+    }
+    split_row_group(is_v ? o.cur_v : o.cur_k, is_v ? o.cur_v_out : o.cur_k_out, rows);
+    return;
+  }
+  const int32_t bh = static_cast<int32_t>(blk / o.slab_chunks);
+  const int32_t chunk = static_cast<int32_t>(blk - static_cast<int64_t>(bh) * o.slab_chunks);
+  WorkItem w;
+  w.b = bh / o.heads;
+  w.h = bh - w.b * o.heads;
+  load_head_segments<256>(o.seg_starts, o.seg_ends, o.seg_counts, o.slab_capacity, o.max_segments, w, seg_start,
+                          seg_pref);
+  const float* const src = (is_v ? o.slab_v : o.slab_k) + w.b * o.slab_capacity * kD;
+  uint8_t* const dst = (is_v ? o.slab_v_out : o.slab_k_out) + w.b * o.slab_capacity * kSRowBytes;
+  int s = 0;  // positions grow, so the segment search walks forward
+  for (int32_t p0 = chunk * kSplitBlockRows; p0 < w.R; p0 += o.slab_chunks * kSplitBlockRows) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int32_t p = p0 + sub + 16 * u;
+      rows[u] = -1;
+      if (p < w.R) {
+        while (seg_pref[s + 1] <= p) ++s;
+        rows[u] = seg_start[s] + (p - seg_pref[s]);
+      }
+    }
+    split_row_group(src, dst, rows);
+  }
 }
 
 template <int VDT>
@@ -442,6 +521,423 @@ __global__ __launch_bounds__(kSThreads, 1) void seg_attn_split_kernel(const int3
                               ring + wave * 32 * kOutPitch);
 }
 
+// ---------------------------------------------------------------- 128-query form
+//
+// The same products and softmax for items of 128 queries: 4 waves x 32
+// queries, two workgroups per CU, and the key stream in 32-key halves (half
+// j = keys 32 (j & 1) .. of tile j >> 1), so that fp32 V fits too: with VDT
+// kSplitRows V arrives as split rows like K, P is split the same way and
+// O += Vh Ph + Vl Ph + Vh Pl (the staged kernel's 2-piece products of fp32 V).
+// Bound by the MFMAs: fp32 V takes 48 of them per half (24 QK, 24 PV) for 114
+// VALU instructions; B = 2, 16 heads, 2304 tokens, budget 0.1 (104 GFLOP
+// nominal, 312 of MFMA): 290 us = 1.07 PFLOP/s of MFMA, with the split of the
+// operands 320 us, against 537 us in the staged kernel (one wave per SIMD,
+// every tile split again for every query tile).
+//  * LDS: two slots each of a K half (hi and lo plane, 16 KiB) and a V half (8
+//    KiB, or 16 KiB with its lo plane): 48 or 64 KiB, so two workgroups share
+//    a CU's 160 KiB.
+//  * Half step j: wait for K(j + 1) and V(j), issued in the step before; one
+//    barrier, which retires every read of K(j) and V(j - 1); issue K(j + 2)
+//    and V(j + 1) into their slots; then half j + 1's QK MFMAs with half j's
+//    exponentials, half j's PV MFMAs with half j + 1's row max.  (Three slots,
+//    the DMAs two steps ahead: 16.7 against 15.8 us at 144 tokens, 32.2 / 31.0
+//    at 576, within 1 % above.)
+constexpr int kHW = 4;                  // waves per workgroup
+constexpr int kHThreads = kHW * 64;
+constexpr int kHKBytes = 32 * kSRowBytes;  // a K half: 16 KiB
+
+template <int VDT>
+struct HalfShape {
+  static constexpr bool kSplitV = VDT == kSplitRows;
+  static constexpr int kVBytes = 32 * kD * 2 * (kSplitV ? 2 : 1);
+  static constexpr int kVRow = kSplitV ? kSRowBytes : kVRowBytes;
+  static constexpr int kRing = 2 * (kHKBytes + kVBytes);
+};
+
+// Two P values per dword rounded to MV, and the bf16 rounding of what that leaves.
+__device__ __forceinline__ uint32_t pack2_rest(float x, float y, uint32_t hi) {
+  const float h0 = __builtin_bit_cast(float, hi << 16);
+  const float h1 = __builtin_bit_cast(float, hi & 0xffff0000u);
+  return pack2<kBF16>(x - h0, y - h1);
+}
+
+// `halves`: the plan's units are items of 256 queries, each run by two
+// workgroups (query halves) with the cut index 2 cut + half.
+template <int VDT>
+__global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32_t* __restrict__ plan_p,
+                                                                    const int32_t n_units, const AttnArgs a,
+                                                                    const Scalars sc, const int32_t n_qt,
+                                                                    const int32_t halves,
+                                                                    const RoundSplit split) {
+  using Shape = HalfShape<VDT>;
+  constexpr bool kSplitV = Shape::kSplitV;
+  constexpr int kThreads = kHThreads;
+  constexpr int kBM = kHW * 32;
+  constexpr int MV = kSplitV ? kBF16 : VDT;
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[Shape::kRing];
+  __shared__ __attribute__((aligned(16))) int32_t rowtab[3][kBN];
+  __shared__ int32_t seg_start[kMaxSegments];
+  __shared__ int32_t seg_pref[kMaxSegments + 1];
+  __shared__ int32_t merge_turn;
+  static_assert(Shape::kRing >= kHW * 32 * kOutPitch, "output staging fits the ring");
+  static_assert(kPartialFloats == 66 * kThreads, "partial record layout");
+
+  // This workgroup's plan unit.  Two workgroups of a 256-query unit sit 8 ids
+  // apart: on one XCD, as the plan dealt the unit.
+  int32_t uid = static_cast<int32_t>(blockIdx.x);
+  int32_t half = 0;
+  if (halves != 0) {
+    half = (uid >> 3) & 1;
+    uid = ((uid >> 4) << 3) + (uid & 7);
+  }
+  int32_t pu[kPlanInts] = {};
+  const bool planned = plan_p != nullptr;
+  if (planned) {
+    if (uid >= n_units) return;
+    const int32_t* src = plan_p + static_cast<int64_t>(uid) * kPlanInts;
+#pragma unroll
+    for (int i = 0; i < kPlanInts; ++i) pu[i] = src[i];
+  }
+  const int64_t cap = a.slab_capacity;
+  const int H = a.heads;
+  const int L = a.cur_len;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform by construction
+  const int g = lane >> 5;
+
+  Unit un{0, 0, 1, 0, 0, 0};
+  WorkItem w;
+  int32_t p0 = 0, p1 = 0;
+  bool cut = false;
+  if (planned) {
+    const int32_t ph = pu[0], pj = pu[1], pcut = pu[4], ppart = pu[5];
+    p0 = pu[2];
+    p1 = pu[3];
+    if (ph < 0 || ph >= H || pj < 0 || pj >= a.batch * n_qt) return;  // not a unit of this launch
+    w.h = ph;
+    w.b = pj / n_qt;
+    w.qt = pj - w.b * n_qt;
+    if (halves != 0) {
+      w.qt = 2 * w.qt + half;
+      if (w.qt * kBM >= L) return;  // no queries in this half (both parts of a cut item leave)
+    }
+    w.bh = w.b * H + w.h;
+    const int32_t c = halves != 0 ? 2 * pcut + half : pcut;
+    cut = pcut >= 0 && a.workspace != nullptr && c < a.ws_cuts && ppart >= 0 && ppart < 2;
+    un.part = cut ? ppart : 0;
+    un.parts = cut ? 2 : 1;
+    un.record = cut ? 2 * c : 0;
+    un.counter = cut ? c : 0;
+    un.arrive = cut && pu[7] != 0 ? 1 : 0;
+  } else {
+    un = split_unit(split, uid);
+    if (split.two == 0) un.item = xcd_item(un.item, a.batch * H, n_qt);
+    int32_t* head_rows = reinterpret_cast<int32_t*>(ring);
+    w = plan_work<kThreads>(a.seg_starts, a.seg_ends, a.seg_counts, cap, H, a.max_segments, a.batch, n_qt,
+                            head_rows, head_rows + kMaxHeads, seg_start, seg_pref, un.item,
+                            head_rows + 2 * kMaxHeads, Shape::kRing / 4 - 2 * kMaxHeads);
+  }
+
+  // Descriptors: split K rows and V rows of the slab (batch row b) and of the
+  // current scale (b, h).
+  const int64_t cur_row0 = static_cast<int64_t>(w.bh) * L;
+  const int32_t ntc = (L + kBN - 1) / kBN;
+  const u32x4_t dk_prior = make_desc(static_cast<const uint8_t*>(a.slab_k) + w.b * cap * kSRowBytes,
+                                     static_cast<uint32_t>(cap * kSRowBytes));
+  const u32x4_t dv_prior = make_desc(static_cast<const uint8_t*>(a.slab_v) + w.b * cap * Shape::kVRow,
+                                     static_cast<uint32_t>(cap * Shape::kVRow));
+  const u32x4_t dk_cur = make_desc(static_cast<const uint8_t*>(a.cur_k) + cur_row0 * kSRowBytes,
+                                   static_cast<uint32_t>(L) * kSRowBytes);
+  const u32x4_t dv_cur = make_desc(static_cast<const uint8_t*>(a.cur_v) + cur_row0 * Shape::kVRow,
+                                   static_cast<uint32_t>(L) * Shape::kVRow);
+
+  // This wave's DMA share of a half: K blocks 4 wave .. + 3 (8 of the hi
+  // plane, 8 of the lo plane; 32 key rows x 32 bytes each) and V chunks 2
+  // wave, 2 wave + 1 (8 key rows x 128 bytes) of each plane.
+  const int k_key = lane & 31;
+  const int k_col = (wave >> 1) * (kD * 2) + (wave & 1) * 128 + (lane >> 5) * 16;
+  const int lp = lane & 31;
+  const int v_key = 16 * (wave >> 1) + 8 * (wave & 1) + 4 * (lp >> 4) + ((lp & 7) >> 1);
+  const int v_col = 2 * ((lane >> 5) * 32 + 16 * ((lp >> 3) & 1) + 8 * (lp & 1));
+  const uint32_t ring_lds = lds_address(ring);
+
+  auto issue_k = [&](int j) {
+    const uint32_t dst = ring_lds + (j & 1) * kHKBytes + wave * 4 * 1024;
+    const int T = j >> 1;
+    int32_t off;
+    u32x4_t d;
+    if (T < ntc) {
+      off = (j * 32 + k_key) * kSRowBytes + k_col;
+      d = dk_cur;
+    } else {
+      const int32_t row = rowtab[(T - ntc) % 3][(j & 1) * 32 + k_key];
+      off = row < 0 ? kPastEnd : row * kSRowBytes + k_col;
+      d = dk_prior;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) dma16(d, dst + i * 1024, off + i * 32);
+  };
+  auto issue_v = [&](int j) {
+    const uint32_t dst = ring_lds + 2 * kHKBytes + (j & 1) * Shape::kVBytes + wave * 2 * 1024;
+    const int T = j >> 1;
+    int32_t off;
+    u32x4_t d;
+    if (T < ntc) {
+      off = (j * 32 + v_key) * Shape::kVRow + v_col;
+      d = dv_cur;
+    } else {
+      const int32_t row = rowtab[(T - ntc) % 3][(j & 1) * 32 + v_key];
+      off = row < 0 ? kPastEnd : row * Shape::kVRow + v_col;
+      d = dv_prior;
+    }
+    dma16(d, dst, off);
+    dma16(d, dst + 1024, off + 128);
+    if constexpr (kSplitV) {
+      dma16(d, dst + 32 * kD * 2, off + kD * 2);
+      dma16(d, dst + 32 * kD * 2 + 1024, off + kD * 2 + 128);
+    }
+  };
+  // A unit whose first tile is a current-scale one (every whole item, and a
+  // part that starts there) issues it, and Q, before the head's tables load:
+  // tables, tile and Q arrive in one round trip.
+  const int32_t first = cut ? (p0 < 0 ? 0 : p0) : 0;
+  const bool early = planned && first < ntc;
+  auto issue_first = [&](int j) {
+    issue_k(j);
+    issue_v(j);
+    issue_k(j + 1);
+  };
+  if (early) issue_first(2 * first);
+
+  // Q in two bf16 pieces: B operands of S^T = K Q^T (query row, d = 16ks +
+  // 8g .. +7); in flight while the tables load
+  const int32_t qrow = w.qt * kBM + wave * 32 + (lane & 31);
+  u32x4_t qh[8], ql[8];
+  {
+    const __amdgpu_buffer_rsrc_t rq = make_rsrc(static_cast<const uint8_t*>(a.q) + cur_row0 * kD * 4,
+                                                static_cast<uint32_t>(L * kD * 4));
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks)
+      load8_split(rq, qrow < L ? (qrow * kD + ks * 16 + g * 8) * 4 : -1, qh[ks], ql[ks]);
+  }
+  if (planned)
+    load_head_segments<kThreads>(a.seg_starts, a.seg_ends, a.seg_counts, cap, a.max_segments, w, seg_start,
+                                 seg_pref);
+  const int32_t R = w.R;
+  const int32_t ntiles = (R + kBN - 1) / kBN + ntc;
+  int32_t parts = un.parts;
+  int32_t tb = 0, te = ntiles;
+  if (planned) {
+    if (cut) {
+      tb = p0 < 0 ? 0 : (p0 > ntiles ? ntiles : p0);
+      te = p1 < tb ? tb : (p1 > ntiles ? ntiles : p1);
+    }
+  } else {
+    // as in the 16-bit kernel: a part needs kMinPartTiles tiles, parts past
+    // the count leave at once
+    parts = ntiles / kMinPartTiles;
+    parts = parts < 1 ? 1 : (parts < un.parts ? parts : un.parts);
+    if (un.part >= parts) return;
+    tb = un.part * ntiles / parts;
+    te = (un.part + 1) * ntiles / parts;
+  }
+  if (tb >= te) {
+    // a planned part with no key tiles (a plan that does not match these
+    // tables): its record is empty -- zero weight in the merge
+    wait_vmcnt<0>();  // an early tile lands before the LDS is used again
+    f32x16_t none[4] = {};
+    merge_parts<kF32, kThreads>(a, sc, un, parts, none, -1e30f, 0.f, w, qrow, L, H, g, merge_turn,
+                                ring + wave * 32 * kOutPitch);
+    return;
+  }
+
+  auto valid_of = [&](int T) { return T < ntc ? min(kBN, L - T * kBN) : min(kBN, R - (T - ntc) * kBN); };
+  int cur_seg = 0;
+  auto fill = [&](int T) {  // wave 0: row table of tile T (a prior-row tile)
+    if (T >= ntc && T < te)
+      fill_rowtab<1>(T - ntc, rowtab[(T - ntc) % 3], cur_seg, w.nseg, R, seg_start, seg_pref, -1);
+  };
+
+  const int j0 = 2 * tb;
+  const int jend = 2 * te;
+  if (wave == 0) {
+    fill(tb);
+    fill(tb + 1);
+  }
+  __syncthreads();
+  if (!early) issue_first(j0);
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) {
+    qh[ks] ^= sc.q_sign;
+    ql[ks] ^= sc.q_sign;
+  }
+
+  f32x16_t oacc[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) oacc[i] = f32x16_t{};
+  float m_run = -1e30f;
+  float l_run = 0.f;
+
+  // S^T of half j from its slot
+  auto qk = [&](f32x16_t& s, int j) {
+    const uint8_t* kst = ring + (j & 1) * kHKBytes + lane * 16;
+    s = f32x16_t{};
+#pragma unroll
+    for (int ks = 0; ks < 8; ++ks) {
+      const u32x4_t kh = *reinterpret_cast<const u32x4_t*>(kst + ks * 1024);
+      const u32x4_t kl = *reinterpret_cast<const u32x4_t*>(kst + (8 + ks) * 1024);
+      s = mfma32<kBF16>(kh, qh[ks], s);
+      s = mfma32<kBF16>(kh, ql[ks], s);
+      s = mfma32<kBF16>(kl, qh[ks], s);
+    }
+  };
+  // O^T += V^T P^T over half j's keys
+  auto pv = [&](const f32x16_t& s, int j) {
+    const uint8_t* vst = ring + 2 * kHKBytes + (j & 1) * Shape::kVBytes + lane * 8;
+#pragma unroll
+    for (int ul = 0; ul < 2; ++ul) {
+      u32x4_t ph, pl;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        ph[i] = pack2<MV>(s[8 * ul + 2 * i], s[8 * ul + 2 * i + 1]);
+        if constexpr (kSplitV) pl[i] = pack2_rest(s[8 * ul + 2 * i], s[8 * ul + 2 * i + 1], ph[i]);
+      }
+#pragma unroll
+      for (int db = 0; db < 4; ++db) {
+        const uint8_t* const blk = vst + ul * 4096 + (db >> 1) * 1024 + (db & 1) * 512;
+        const u32x2_t lo = ds_read_tr(blk);
+        const u32x2_t hi = ds_read_tr(blk + 2048);
+        const u32x4_t vh = {lo[0], lo[1], hi[0], hi[1]};
+        oacc[db] = mfma32<MV>(vh, ph, oacc[db]);
+        if constexpr (kSplitV) {
+          const u32x2_t lo2 = ds_read_tr(blk + 32 * kD * 2);
+          const u32x2_t hi2 = ds_read_tr(blk + 32 * kD * 2 + 2048);
+          const u32x4_t vl = {lo2[0], lo2[1], hi2[0], hi2[1]};
+          oacc[db] = mfma32<MV>(vh, pl, oacc[db]);
+          oacc[db] = mfma32<MV>(vl, ph, oacc[db]);
+        }
+      }
+    }
+  };
+  auto masked_max = [&](f32x16_t& s, int j) {
+    float mx = half_max(s);
+    asm volatile("" : "+v"(mx));
+    const int v = valid_of(j >> 1);
+    if (v < 32 * ((j & 1) + 1)) {
+      mask_half(s, j & 1, v, g);
+      mx = half_max(s);
+    }
+    return mx;
+  };
+
+  // Prologue: every issued half landed; S of the first half and its max.
+  wait_vmcnt<0>();
+  __syncthreads();
+  f32x16_t sa, sb;
+  qk(sa, j0);
+  move_max(oacc, m_run, l_run, masked_max(sa, j0), sc.c, sc.thresh);
+
+  // Half step j: scur = S(j) (max applied), snext receives S(j + 1) unless j
+  // is the item's last half.
+  auto step = [&](auto more_tag, f32x16_t& scur, f32x16_t& snext, int j) {
+    constexpr bool kMore = decltype(more_tag)::value;
+    wait_vmcnt<0>();  // this wave's share of K(j + 1) and V(j)
+    __syncthreads();
+    if constexpr (kMore) {
+      if (j + 2 < jend) issue_k(j + 2);
+      issue_v(j + 1);
+    }
+    // the table of the tile whose K is first issued in the next step
+    if (wave == 0 && (j & 1) != 0) fill((j + 3) >> 1);
+    if constexpr (kMore) qk(snext, j + 1);
+    exp_half(scur, m_run, sc.c, l_run);
+    pv(scur, j);
+    if constexpr (kMore) {
+      asm volatile("" : "+v"(l_run));
+      move_max(oacc, m_run, l_run, masked_max(snext, j + 1), sc.c, sc.thresh);
+    }
+  };
+  using More = std::integral_constant<bool, true>;
+  using Last = std::integral_constant<bool, false>;
+  int j = j0;
+  for (; j + 2 < jend; j += 2) {
+    step(More{}, sa, sb, j);
+    step(More{}, sb, sa, j + 1);
+  }
+  step(More{}, sa, sb, j);
+  step(Last{}, sb, sa, j + 1);
+
+  if (parts == 1) {
+    if (a.out_dtype != kF32 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0) {
+      __syncthreads();  // every wave is past its last half: the ring is free
+      uint8_t* const stage = ring + wave * 32 * kOutPitch;
+      const int32_t qrow0 = w.qt * kBM + wave * 32;
+      if (a.out_dtype == kF16)
+        write_output_lds<kF16>(oacc, m_run, l_run, sc.c, a.out, a.lse, w.b, w.h, qrow0, L, H, w.bh, lane, stage);
+      else
+        write_output_lds<kBF16>(oacc, m_run, l_run, sc.c, a.out, a.lse, w.b, w.h, qrow0, L, H, w.bh, lane, stage);
+    } else {
+      write_output(oacc, m_run, l_run, sc.c, a.out, a.lse, w.b, w.h, qrow, L, H, w.bh, g, a.out_dtype);
+    }
+    return;
+  }
+  merge_parts<kF32, kThreads>(a, sc, un, parts, oacc, m_run, l_run, w, qrow, L, H, g, merge_turn,
+                              ring + wave * 32 * kOutPitch);
+}
+
+template <int VDT>
+hipError_t launch_half(const AttnArgs& a, const Scalars& s, hipStream_t st, int32_t plan_queries) {
+  const int32_t n_qt = (a.cur_len + 127) / 128;
+  const int64_t items = static_cast<int64_t>(a.batch) * a.heads * n_qt;
+  if (items <= 0) return hipSuccess;
+  if (items > 0x3fffffffLL) return hipErrorInvalidConfiguration;
+  int device = 0;
+  const int32_t slots = a.workspace != nullptr && hipGetDevice(&device) == hipSuccess ? split_slots(device) : 0;
+  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0};
+  if (slots > 0 && a.workspace_bytes >= split_workspace_bytes(slots))
+    split = round_split(static_cast<int32_t>(items), slots, (a.cur_len + kBN - 1) / kBN);
+  AttnArgs b = a;
+  b.ws_cuts = 0;
+  if (a.workspace != nullptr && a.workspace_bytes > kCounterBytes) {
+    const int64_t by_records = (a.workspace_bytes - kCounterBytes) / (2LL * kPartialFloats * 4);
+    b.ws_cuts = static_cast<int32_t>(by_records < kMaxCounters ? by_records : kMaxCounters);
+  }
+  const bool halves = a.plan != nullptr && plan_queries == kSBM;
+  int64_t grid = a.plan != nullptr ? a.plan_units : split_units(split);
+  if (halves) grid = (grid + 7) / 8 * 16;
+  if (grid <= 0) return hipSuccess;
+  if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  seg_attn_half_kernel<VDT><<<dim3(static_cast<uint32_t>(grid)), kHThreads, 0, st>>>(
+      b.plan, b.plan != nullptr ? b.plan_units : 0, b, s, halves ? (a.cur_len + kSBM - 1) / kSBM : n_qt,
+      halves ? 1 : 0, split);
+  return hipGetLastError();
+}
+
+// Whether a call on split K rows with 16-bit V runs as 128-query workgroups
+// (seg_attn_half_kernel; a plan's 256-query units as two halves each) instead
+// of 256-query ones.  The 8-wave form is the faster one once every CU has its
+// fill of it (546 against 592 us on the 2B final step, 512 items of 256
+// queries; 198 / 204 at 288 items), the halves before that: they spread over
+// twice the workgroups, a last tile of at most 128 queries costs half, and a
+// call without a plan cuts its items in two (one image pair, 16 heads, us,
+// halves / 8 waves at 144, 400, 576, 1024, 1600, 2304 tokens: planned 16.1 /
+// 19.5, 25.7 / 33.0, 30.7 / 39.9, 59.2 / 63.6, 105.0 / 107.1, 204 / 198; not
+// planned 17.2 / 20.4, 26.9 / 33.8, 37.0 / 47.2, 58.5 / 96.9, 105.7 / 126,
+// 203 / 229; not planned 4096 tokens 613 / 587).  So: up to one 256-query
+// item per CU (below two without a plan), or where half tiles save at least
+// an eighth of the padded queries (576 tokens, 768 items: 135 / 143 us; 1600
+// tokens save 7 %: 771 / 753).
+bool split_in_halves(const AttnArgs& a) {
+  int device = 0;
+  const int32_t cus = hipGetDevice(&device) == hipSuccess ? split_slots(device) / 2 : 0;
+  const int64_t t256 = (static_cast<int64_t>(a.cur_len) + kSBM - 1) / kSBM;
+  const int64_t t128 = (static_cast<int64_t>(a.cur_len) + 127) / 128;
+  const int64_t items = static_cast<int64_t>(a.batch) * a.heads * t256;
+  if (a.plan != nullptr ? items <= cus : items < 2 * static_cast<int64_t>(cus)) return true;
+  return 8 * t128 <= 7 * 2 * t256;
+}
+
 template <int VDT>
 hipError_t launch(const AttnArgs& a, const Scalars& s, hipStream_t st) {
   const int32_t n_qt = (a.cur_len + kSBM - 1) / kSBM;
@@ -470,8 +966,28 @@ bool attention_split_supported(const AttnArgs& a) {
 }
 
 hipError_t launch_attention_split(const AttnArgs& a, const attn::Scalars& s, hipStream_t stream) {
+  if (a.v_dtype == kSplitRows) {  // only from hkv_segmented_attention_split: plans of 128-query items
+    if (a.q_dtype != kF32 || a.k_dtype != kSplitRows) return hipErrorInvalidValue;
+    return launch_half<kSplitRows>(a, s, stream, 128);
+  }
   if (!attention_split_supported(a)) return hipErrorInvalidValue;
+  if (split_in_halves(a))
+    return a.v_dtype == kBF16 ? launch_half<kBF16>(a, s, stream, kSBM) : launch_half<kF16>(a, s, stream, kSBM);
   return a.v_dtype == kBF16 ? launch<kBF16>(a, s, stream) : launch<kF16>(a, s, stream);
+}
+
+hipError_t launch_split_operands(SplitOperands o, bool with_v, hipStream_t stream) {
+  const int64_t cur_blocks = (o.cur_rows + kSplitBlockRows - 1) / kSplitBlockRows;
+  const int64_t bh = static_cast<int64_t>(o.batch) * o.heads;
+  const int64_t share = kSplitSlabBlocks / bh < 4 ? 4 : kSplitSlabBlocks / bh;
+  const int64_t chunks = (o.slab_capacity + kSplitBlockRows - 1) / kSplitBlockRows;
+  o.slab_chunks = static_cast<int32_t>(chunks < share ? chunks : share);
+  o.slab_blocks = o.max_segments > 0 ? bh * o.slab_chunks : 0;
+  const int64_t blocks = cur_blocks + o.slab_blocks;
+  if (blocks <= 0) return hipSuccess;
+  if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  split_operands_kernel<<<dim3(static_cast<uint32_t>(blocks), with_v ? 2 : 1), 256, 0, stream>>>(o);
+  return hipGetLastError();
 }
 
 hipError_t launch_split_rows(const float* src, void* dst, int64_t rows, hipStream_t stream) {

@@ -131,14 +131,37 @@ def segmented_attention_plan(segment_starts, segment_ends, segment_counts, *, ba
     return out
 
 
+def _split_rows_enabled() -> bool:
+    return _lib.env_get("HKV_ATTN_SPLIT_ROWS", "1").strip().lower() not in {"0", "false", "no", "off"}
+
+
 def _split_rows_path(q_dtype, k_dtype, v_dtype, qk_mode: int, value_mode: int) -> bool:
     """fp32 q/k with 16-bit v at dot modes other than fp32 run the split-row
     kernel: K is first written as split rows (hkv_split_rows).  HKV_ATTN_SPLIT_ROWS=0
     keeps them on the register-staged kernel (for comparisons)."""
-    if _lib.env_get("HKV_ATTN_SPLIT_ROWS", "1").strip().lower() in {"0", "false", "no", "off"}:
+    if not _split_rows_enabled():
         return False
     return (q_dtype == torch.float32 and k_dtype == torch.float32 and v_dtype in (torch.float16, torch.bfloat16)
             and qk_mode != 2 and value_mode != 2)
+
+
+# Current rows (batch x heads x length) from which all-fp32 calls split K and V
+# ahead of the attention.  The split-row kernel is the faster one at every size
+# (one image pair, 16 heads, device us with the split launch / staged kernel:
+# 36 tokens 16.3 / 16.8, 144: 27.3 / 29.2, 1024: 96 / 136, 2304: 320 / 537),
+# but below this a call is bound by its host work, which the split adds to
+# (a scratch tensor and a second launch, ~4 us).
+_SPLIT_VALUES_ROWS = 4096
+
+
+def _split_values_path(q, k, v, qk_mode: int, value_mode: int) -> bool:
+    """fp32 q, k and v at the default (or tf32) dot modes, with enough rows, run
+    the split-row kernel's 128-query form on split copies of K and V; otherwise
+    (and with HKV_ATTN_SPLIT_ROWS=0) the register-staged kernel, which splits
+    every tile for every query tile itself."""
+    return (q.dtype == torch.float32 and k.dtype == torch.float32 and v.dtype == torch.float32
+            and qk_mode != 2 and value_mode != 2
+            and q.shape[0] * q.shape[1] * q.shape[2] >= _SPLIT_VALUES_ROWS and _split_rows_enabled())
 
 
 def split_rows_k_format(q_dtype, k_dtype, v_dtype) -> bool:
@@ -231,11 +254,15 @@ def attention_fuses_append(q_dtype, k_dtype, v_dtype, *, k_split_rows: bool = Fa
     return not _split_rows_path(qd, kd, v_dtype, qk_mode, value_mode)
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """``t``, or a copy of it where it does not start on a 16-byte boundary."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _split_rows(t: torch.Tensor, stream) -> torch.Tensor:
     """fp32 ``[..., 128]`` rows as split rows ``[..., 256]`` bf16 (128 high
     parts, then 128 low parts), by the HIP kernel ``hkv_split_rows``."""
-    if t.data_ptr() % 16 != 0:
-        t = t.clone()
+    t = _aligned(t)
     out = torch.empty(tuple(t.shape[:-1]) + (2 * t.shape[-1],), device=t.device, dtype=torch.bfloat16)
     rows = t.numel() // t.shape[-1]
     if rows > 0:
@@ -517,6 +544,7 @@ def fused_real_pruning_flat_segmented_attention(
     if k_split_rows:
         _check_split_rows_k(q.dtype, current_k.dtype, current_v.dtype, qk_mode, value_mode)
     split = k_split_rows or _split_rows_path(q.dtype, current_k.dtype, current_v.dtype, qk_mode, value_mode)
+    split_v = not split and _split_values_path(q, current_k, current_v, qk_mode, value_mode)
     if work_plan is not None:
         if (work_plan.dtype != torch.int32 or work_plan.ndim != 2 or work_plan.shape[1] != PLAN_INTS
                 or not work_plan.is_contiguous()):
@@ -564,14 +592,26 @@ def fused_real_pruning_flat_segmented_attention(
         offsets2 = offsets2.contiguous()
     stream = torch.cuda.current_stream(q.device)
     ws = _lib.attention_workspace(q.device, stream)
-    k_code = _lib.dtype_code(current_k.dtype)
-    converted = promoted or (split and not k_split_rows)
-    if split:
-        # fp32 K as split rows for the split-row kernel (the q split happens in it)
-        if not k_split_rows:
-            persisted_k = _split_rows(persisted_k, stream)
-            current_k = _split_rows(current_k, stream)
-        k_code = _lib.DTYPE_SPLIT_ROWS
+    k_code = _lib.DTYPE_SPLIT_ROWS if k_split_rows else _lib.dtype_code(current_k.dtype)
+    # fp32 K (and V) rows go to the split-row kernels as split copies made by
+    # the same call (the q split happens in the kernel)
+    splits = (split and not k_split_rows) or split_v
+    converted = promoted or splits
+    lib = _lib.load()
+    scratch = None
+    if splits:
+        # the split reads 16 bytes per access (a slab that the append writes
+        # stays itself: the library refuses it when it is not aligned)
+        current_k = _aligned(current_k)
+        persisted_k = persisted_k if append_offsets is not None else _aligned(persisted_k)
+        if split_v:
+            current_v = _aligned(current_v)
+            persisted_v = persisted_v if append_offsets is not None else _aligned(persisted_v)
+        need = int(lib.hkv_segmented_attention_split_bytes(batch_size, num_heads, current_len,
+                                                           int(persisted_k.shape[1]),
+                                                           _lib.dtype_code(current_v.dtype)))
+        _lib.check(min(need, 0))
+        scratch = torch.empty((need,), device=q.device, dtype=torch.uint8)
     args = [
         q.data_ptr(), persisted_k.data_ptr(), persisted_v.data_ptr(),
         segment_starts.data_ptr(), segment_ends.data_ptr(), segment_counts.data_ptr(),
@@ -585,8 +625,13 @@ def fused_real_pruning_flat_segmented_attention(
         int(work_plan.shape[0]) if work_plan is not None else 0,
         ws.data_ptr() if ws is not None else None, int(ws.numel()) if ws is not None else 0,
     ]
-    lib = _lib.load()
-    if append_offsets is None:
+    if splits:
+        fn = lib.hkv_segmented_attention_split
+        args.append(append_offsets.data_ptr() if append_offsets is not None else None)
+        args += ([None, None, 0, None] if append_also is None else
+                 [slab2_k.data_ptr(), slab2_v.data_ptr(), int(slab2_k.shape[1]), offsets2.data_ptr()])
+        args += [scratch.data_ptr(), int(scratch.numel())]
+    elif append_offsets is None:
         fn = lib.hkv_segmented_attention
     elif append_also is None:
         fn = lib.hkv_segmented_attention_append

@@ -220,6 +220,33 @@ int32_t hkv_segmented_attention_append2(const void* q, void* slab_k, void* slab_
                                         const int32_t* append_offsets, void* slab2_k, void* slab2_v,
                                         int64_t slab2_capacity, const int32_t* append2_offsets, void* stream);
 
+/*
+ * hkv_segmented_attention_append2 on float32 q and k (v float32 or 16-bit,
+ * default or tf32 dot modes) that first writes the operands the split-row
+ * kernels read: the current rows, and the slab rows that the tables hold, of
+ * K (and of float32 V) as split rows in `scratch` (one launch), then the
+ * attention on them, then the append of the float32 rows themselves (a launch
+ * of its own).  append_offsets and the second destination may be NULL as in
+ * the calls above; work_plan items are 256 queries for 16-bit v and 128 for
+ * float32 v (hkv_segmented_attention_item_shape).  float32 tensors and scratch
+ * 16-byte aligned; scratch of at least hkv_segmented_attention_split_bytes()
+ * bytes, in use until the launches are done.  No counterpart in the reference,
+ * whose Triton dot takes fp32 operands as they are.
+ */
+int64_t hkv_segmented_attention_split_bytes(int32_t batch, int32_t heads, int32_t cur_len, int64_t slab_capacity,
+                                            int32_t v_dtype);
+int32_t hkv_segmented_attention_split(const void* q, void* slab_k, void* slab_v, const int32_t* seg_starts,
+                                      const int32_t* seg_ends, const int32_t* seg_counts, const void* cur_k,
+                                      const void* cur_v, void* out, float* lse, int32_t batch, int32_t heads,
+                                      int32_t cur_len, int64_t slab_capacity, int32_t max_segments,
+                                      int32_t head_dim, int32_t q_dtype, int32_t k_dtype, int32_t v_dtype,
+                                      int32_t out_dtype, float softmax_scale, int32_t use_exp2, int32_t qk_dot_mode,
+                                      int32_t value_dot_mode, const int32_t* work_plan, int32_t plan_units,
+                                      void* workspace, int64_t workspace_bytes, const int32_t* append_offsets,
+                                      void* slab2_k, void* slab2_v, int64_t slab2_capacity,
+                                      const int32_t* append2_offsets, void* scratch, int64_t scratch_bytes,
+                                      void* stream);
+
 /* A bound attention call: hkv_segmented_attention_append's arguments other
  * than the tensors (tables, shapes, dtypes, scale, dot modes, work plan,
  * workspace and append offsets) validated once into a caller-owned block of
