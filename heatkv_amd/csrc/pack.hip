@@ -9,21 +9,30 @@
 // pointers and row pitch allow it (128-bit loads and stores), else in 4- or
 // 2-byte words.  The copy is bit-exact by construction.
 //
-// Work split: one workgroup of 256 threads per (item, 64-row chunk, batch
-// row).  For bf16 D=128 a chunk is 16 KiB of K plus 16 KiB of V, four
-// independent 16-byte loads in flight per thread per tensor.  Workgroups whose
-// chunk lies beyond their item's length exit at once (append items all share
-// one length, so none are idle there).
+// Work split: one workgroup of 256 threads per (item, 16-row chunk, batch
+// row).  For bf16 D=128 a chunk is 4 KiB of K plus 4 KiB of V: one 16-byte load
+// of each tensor per thread, both in flight together, and many short workgroups
+// per CU.  Deeper batches per thread are slower (one plain copy of 604 MB, 1 / 2
+// / 4 / 8 vectors per thread: 6.6 / 6.1 / 6.3 / 4.4 TB/s), and loads and stores
+// are non-temporal (stream_mem.h).  B=8, 32 items of 2304 bf16 rows (604 MB
+// moved): 108.8 us with 64-row chunks, K before V and ordinary accesses, 95.5 us
+// now (6.3 TB/s; non-temporal loads or stores alone 102, neither 106).  B=2, 16
+// items: 2304 rows 12.5 / 12.4 us, 576 rows 4.6 / 3.8, 64 rows 3.4 / 2.4.
+// Workgroups whose chunk lies beyond their item's length exit at once (append
+// items all share one length, so none are idle there).
 #include "hkv_internal.h"
+#include "stream_mem.h"
 
 namespace hkv {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kChunkRows = 64;
+constexpr int kChunkRows = 16;
+constexpr int kChunkRowsWide = 64;  // where 16-row chunks would be more workgroups than a launch takes
+constexpr int64_t kMaxBlocks = 0xffffffffLL / kThreads;  // a launch has fewer than 2^32 threads in x
 constexpr int kUnroll = 4;
 
-struct alignas(16) U16B { uint32_t w[4]; };
+typedef uint32_t U16B __attribute__((ext_vector_type(4)));
 
 template <typename U>
 __device__ __forceinline__ void copy_range(char* __restrict__ dst, const char* __restrict__ src,
@@ -43,8 +52,29 @@ __device__ __forceinline__ void copy_range(char* __restrict__ dst, const char* _
   for (; i < n; i += kThreads) d[i] = s[i];
 }
 
+// Two ranges, one vector of each in flight per thread.
 template <typename UK, typename UV>
-__global__ __launch_bounds__(kThreads) void pack_kernel(PackArgs a, int32_t chunks) {
+__device__ __forceinline__ void copy_ranges(char* __restrict__ dst_k, const char* __restrict__ src_k, int64_t k_bytes,
+                                            char* __restrict__ dst_v, const char* __restrict__ src_v,
+                                            int64_t v_bytes) {
+  const int64_t nk = k_bytes / static_cast<int64_t>(sizeof(UK)), nv = v_bytes / static_cast<int64_t>(sizeof(UV));
+  UK* dk = reinterpret_cast<UK*>(dst_k);
+  UV* dv = reinterpret_cast<UV*>(dst_v);
+  const UK* sk = reinterpret_cast<const UK*>(src_k);
+  const UV* sv = reinterpret_cast<const UV*>(src_v);
+  const int64_t n = nk > nv ? nk : nv;
+  for (int64_t i = threadIdx.x; i < n; i += kThreads) {
+    UK xk{};
+    UV xv{};
+    if (i < nk) xk = stream_load(sk + i);
+    if (i < nv) xv = stream_load(sv + i);
+    if (i < nk) stream_store(dk + i, xk);
+    if (i < nv) stream_store(dv + i, xv);
+  }
+}
+
+template <typename UK, typename UV>
+__global__ __launch_bounds__(kThreads) void pack_kernel(PackArgs a, int32_t chunks, int32_t chunk_rows) {
   const int32_t item = blockIdx.x / chunks;
   const int32_t chunk = blockIdx.x - item * chunks;
   const int64_t b = blockIdx.y;
@@ -56,9 +86,9 @@ __global__ __launch_bounds__(kThreads) void pack_kernel(PackArgs a, int32_t chun
   const int64_t dst_start = a.dst_starts[item];
   asm volatile("" : "+s"(len) : "s"(src_start), "s"(dst_start));
   if (len > a.row_limit) len = a.row_limit;
-  const int64_t r0 = static_cast<int64_t>(chunk) * kChunkRows;
+  const int64_t r0 = static_cast<int64_t>(chunk) * chunk_rows;
   if (r0 >= len) return;
-  const int64_t r1 = (r0 + kChunkRows < len) ? r0 + kChunkRows : len;
+  const int64_t r1 = (r0 + chunk_rows < len) ? r0 + chunk_rows : len;
   const int64_t s0 = src_start + r0;
   const int64_t d0 = dst_start + r0;
   // Clip the row range so that both the source and the destination row stay
@@ -74,12 +104,10 @@ __global__ __launch_bounds__(kThreads) void pack_kernel(PackArgs a, int32_t chun
   const int64_t D = a.head_dim;
   const int64_t src_elem = b * a.src_batch_stride + (s0 + lo) * D;
   const int64_t dst_elem = b * a.dst_batch_stride + (d0 + lo) * D;
-  copy_range<UK>(static_cast<char*>(a.dst_k) + dst_elem * a.k_elem_bytes,
-                 static_cast<const char*>(a.src_k) + src_elem * a.k_elem_bytes,
-                 rows * D * a.k_elem_bytes);
-  copy_range<UV>(static_cast<char*>(a.dst_v) + dst_elem * a.v_elem_bytes,
-                 static_cast<const char*>(a.src_v) + src_elem * a.v_elem_bytes,
-                 rows * D * a.v_elem_bytes);
+  copy_ranges<UK, UV>(static_cast<char*>(a.dst_k) + dst_elem * a.k_elem_bytes,
+                      static_cast<const char*>(a.src_k) + src_elem * a.k_elem_bytes, rows * D * a.k_elem_bytes,
+                      static_cast<char*>(a.dst_v) + dst_elem * a.v_elem_bytes,
+                      static_cast<const char*>(a.src_v) + src_elem * a.v_elem_bytes, rows * D * a.v_elem_bytes);
 }
 
 // Widest copy unit (16, 4 or 2 bytes) that keeps every access aligned.
@@ -98,11 +126,11 @@ int unit_bytes(const void* src, const void* dst, int64_t src_bs, int64_t dst_bs,
 }
 
 template <typename UK>
-hipError_t launch_v(const PackArgs& a, int uv, dim3 grid, int32_t chunks, hipStream_t st) {
+hipError_t launch_v(const PackArgs& a, int uv, dim3 grid, int32_t chunks, int32_t chunk_rows, hipStream_t st) {
   switch (uv) {
-    case 16: pack_kernel<UK, U16B><<<grid, kThreads, 0, st>>>(a, chunks); break;
-    case 4: pack_kernel<UK, uint32_t><<<grid, kThreads, 0, st>>>(a, chunks); break;
-    default: pack_kernel<UK, uint16_t><<<grid, kThreads, 0, st>>>(a, chunks); break;
+    case 16: pack_kernel<UK, U16B><<<grid, kThreads, 0, st>>>(a, chunks, chunk_rows); break;
+    case 4: pack_kernel<UK, uint32_t><<<grid, kThreads, 0, st>>>(a, chunks, chunk_rows); break;
+    default: pack_kernel<UK, uint16_t><<<grid, kThreads, 0, st>>>(a, chunks, chunk_rows); break;
   }
   return hipGetLastError();
 }
@@ -150,7 +178,10 @@ hipError_t launch_concat(const ConcatArgs& a, hipStream_t stream) {
 
 hipError_t launch_pack(const PackArgs& a, hipStream_t stream) {
   if (a.n_items <= 0 || a.row_limit <= 0 || a.batch <= 0) return hipSuccess;
-  const int64_t chunks64 = (static_cast<int64_t>(a.row_limit) + kChunkRows - 1) / kChunkRows;
+  int32_t chunk_rows = kChunkRows;
+  auto count = [&] { return (static_cast<int64_t>(a.row_limit) + chunk_rows - 1) / chunk_rows; };
+  if (count() * a.n_items > kMaxBlocks) chunk_rows = kChunkRowsWide;
+  const int64_t chunks64 = count();
   const int64_t blocks = chunks64 * a.n_items;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   const int32_t chunks = static_cast<int32_t>(chunks64);
@@ -160,9 +191,9 @@ hipError_t launch_pack(const PackArgs& a, hipStream_t stream) {
   const int uv = unit_bytes(a.src_v, a.dst_v, a.src_batch_stride, a.dst_batch_stride,
                             a.head_dim, a.v_elem_bytes);
   switch (uk) {
-    case 16: return launch_v<U16B>(a, uv, grid, chunks, stream);
-    case 4: return launch_v<uint32_t>(a, uv, grid, chunks, stream);
-    default: return launch_v<uint16_t>(a, uv, grid, chunks, stream);
+    case 16: return launch_v<U16B>(a, uv, grid, chunks, chunk_rows, stream);
+    case 4: return launch_v<uint32_t>(a, uv, grid, chunks, chunk_rows, stream);
+    default: return launch_v<uint16_t>(a, uv, grid, chunks, chunk_rows, stream);
   }
 }
 
