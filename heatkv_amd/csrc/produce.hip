@@ -30,9 +30,23 @@
 // Work split: 16 lanes per (b, l, h) row, 8 elements (16 bytes of bf16) per
 // lane per tensor; rows in (b, l, h) order, so the 16 rows of a 256-thread
 // workgroup read one token's contiguous q, k and v blocks and each row writes
-// whole 512-byte (fp32) or 256-byte (bf16) output rows.  Pure streaming:
-// 768 bytes read and 1280 bytes written per row with fp32 q/k (HBM bound).
+// whole 512-byte (fp32) or 256-byte (bf16) output rows.  HBM bound, two thirds
+// of it writes (768 bytes read and 1280 written per row with fp32 q/k, 768
+// more where the row is appended), so the writes decide:
+//  * every store instruction fills whole 128-byte lines.  A lane's 8 fp32
+//    values are 32 bytes; stored as two 16-byte pieces each instruction fills
+//    half of every line it touches, so the row is exchanged between its 16
+//    lanes first (lane reads hidden behind memory);
+//  * with whole lines the stores are non-temporal (stream_mem.h).
+// 4096 tokens, B=2, 16 heads, fp32 q, split k rows, appending half the heads,
+// device us with the projection in the last-level cache (as the GEMM before
+// leaves it) / from HBM: 62 / 66 with half-line ordinary stores, 65 / 76
+// half-line non-temporal, 57 / 64 whole-line ordinary, 50 / 60 whole-line
+// non-temporal (6.4 / 5.3 TB/s).  Non-temporal loads as well: 57 / 56.5, so the
+// loads stay ordinary; one head's 16 tokens per workgroup instead: 50 / 61.
+// 1024 tokens: 15.5 / 20 -> 13.1 / 15.6, 256 tokens: 6.5 / 8.0 -> 6.1 / 6.8.
 #include "hkv_internal.h"
+#include "stream_mem.h"
 
 namespace hkv {
 namespace {
@@ -69,8 +83,27 @@ __device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
 }
 
+// Stores the 32-byte pieces (a, b) of a row's 16 lanes, lane j holding bytes
+// 32j .. 32j + 31 of the 512-byte row at `row`, as two instructions of 256
+// contiguous bytes per row: lane j writes bytes 16j and 256 + 16j, which lanes
+// j / 2 and 8 + j / 2 hold.
+__device__ __forceinline__ void store_row_32(uint8_t* row, int j, u32x4_t a, u32x4_t b) {
+  u32x4_t lo, hi;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t a0 = __shfl(a[i], j >> 1, kLanes), b0 = __shfl(b[i], j >> 1, kLanes);
+    const uint32_t a1 = __shfl(a[i], 8 + (j >> 1), kLanes), b1 = __shfl(b[i], 8 + (j >> 1), kLanes);
+    lo[i] = (j & 1) ? b0 : a0;
+    hi[i] = (j & 1) ? b1 : a1;
+  }
+  stream_store(reinterpret_cast<u32x4_t*>(row + j * 16), lo);
+  stream_store(reinterpret_cast<u32x4_t*>(row + 256 + j * 16), hi);
+}
+
+// The row's elements [8j, 8j + 8) of row `row` of `base`; the row's 16 lanes
+// call it together.
 template <int DT>
-__device__ __forceinline__ void store_row8(void* base, int64_t elem, const float (&x)[kPer]) {
+__device__ __forceinline__ void store_row8(void* base, int64_t row_index, int j, const float (&x)[kPer]) {
   if constexpr (DT == kSplitRows) {
     // split row (hkv_split_rows' format, 512 bytes like an fp32 row): the
     // 128 bf16 high parts hi = bf16(x), then the 128 low parts bf16(x - hi)
@@ -82,21 +115,23 @@ __device__ __forceinline__ void store_row8(void* base, int64_t elem, const float
       const float h1 = __builtin_bit_cast(float, hi[k] & 0xffff0000u);
       lo[k] = pack_bf16x2(x[2 * k] - h0, x[2 * k + 1] - h1);
     }
-    uint8_t* const row = static_cast<uint8_t*>(base) + (elem / kD) * (kD * 4) + (elem % kD) * 2;
-    *reinterpret_cast<u32x4_t*>(row) = hi;
-    *reinterpret_cast<u32x4_t*>(row + kD * 2) = lo;
+    uint8_t* const p = static_cast<uint8_t*>(base) + row_index * (kD * 4) + j * (kPer * 2);
+    stream_store(reinterpret_cast<u32x4_t*>(p), hi);
+    stream_store(reinterpret_cast<u32x4_t*>(p + kD * 2), lo);
   } else if constexpr (DT == kF32) {
-    f32x4_t* p = reinterpret_cast<f32x4_t*>(static_cast<float*>(base) + elem);
-    p[0] = f32x4_t{x[0], x[1], x[2], x[3]};
-    p[1] = f32x4_t{x[4], x[5], x[6], x[7]};
-  } else if constexpr (DT == kF16) {
-    u32x4_t w = {pack_f16x2(x[0], x[1]), pack_f16x2(x[2], x[3]), pack_f16x2(x[4], x[5]),
-                 pack_f16x2(x[6], x[7])};
-    *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(base) + elem) = w;
+    u32x4_t a, b;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      a[i] = __float_as_uint(x[i]);
+      b[i] = __float_as_uint(x[4 + i]);
+    }
+    store_row_32(static_cast<uint8_t*>(base) + row_index * (kD * 4), j, a, b);
   } else {
-    u32x4_t w = {pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]),
-                 pack_bf16x2(x[6], x[7])};
-    *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(base) + elem) = w;
+    u32x4_t w;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      w[i] = DT == kF16 ? pack_f16x2(x[2 * i], x[2 * i + 1]) : pack_bf16x2(x[2 * i], x[2 * i + 1]);
+    stream_store(reinterpret_cast<u32x4_t*>(static_cast<uint8_t*>(base) + row_index * (kD * 2) + j * (kPer * 2)), w);
   }
 }
 
@@ -167,13 +202,12 @@ __device__ __forceinline__ void load_row8(const uint8_t* p, float (&x)[kPer], u3
 }
 
 template <int IT>
-__device__ __forceinline__ void store_raw8(void* base, int64_t elem, const u32x4_t (&raw)[2]) {
+__device__ __forceinline__ void store_raw8(void* base, int64_t row_index, int j, const u32x4_t (&raw)[2]) {
   if constexpr (IT == kF32) {
-    u32x4_t* p = reinterpret_cast<u32x4_t*>(static_cast<float*>(base) + elem);
-    p[0] = raw[0];
-    p[1] = raw[1];
+    store_row_32(static_cast<uint8_t*>(base) + row_index * (kD * 4), j, raw[0], raw[1]);
   } else {
-    *reinterpret_cast<u32x4_t*>(static_cast<uint16_t*>(base) + elem) = raw[0];
+    stream_store(reinterpret_cast<u32x4_t*>(static_cast<uint8_t*>(base) + row_index * (kD * 2) + j * (kPer * 2)),
+                 raw[0]);
   }
 }
 
@@ -182,14 +216,15 @@ __device__ __forceinline__ void store_raw8(void* base, int64_t elem, const u32x4
 template <int IT, int QT, int KT = QT>
 __global__ __launch_bounds__(kThreads) void produce_kernel(ProduceArgs a) {
   constexpr int kElem = IT == kF32 ? 4 : 2;
-  const int64_t row = static_cast<int64_t>(blockIdx.x) * kRowsPerBlock + threadIdx.x / kLanes;
+  // (b, l, h); 32-bit, as the launch checks
+  const uint32_t row = blockIdx.x * kRowsPerBlock + threadIdx.x / kLanes;
   const int j = threadIdx.x % kLanes;
-  // Whole 16-lane rows leave together, so the row reductions stay complete.
+  // Whole 16-lane rows leave together, so the row exchanges stay complete.
   if (row >= a.rows) return;
-  const int32_t h = static_cast<int32_t>(row % a.heads);
-  const int64_t tok = row / a.heads;  // b * len + l
-  const int32_t l = static_cast<int32_t>(tok % a.len);
-  const int64_t b = tok / a.len;
+  const int64_t tok = row / static_cast<uint32_t>(a.heads);  // b * len + l
+  const int32_t h = static_cast<int32_t>(row - static_cast<uint32_t>(tok) * a.heads);
+  const int64_t b = static_cast<uint32_t>(tok) / static_cast<uint32_t>(a.len);
+  const int32_t l = static_cast<int32_t>(tok - b * a.len);
   const int64_t hd = static_cast<int64_t>(a.heads) * kD;
 
   const uint8_t* src = static_cast<const uint8_t*>(a.qkv) +
@@ -222,25 +257,25 @@ __global__ __launch_bounds__(kThreads) void produce_kernel(ProduceArgs a) {
     rotate(k, rc, rs);
   }
 
-  const int64_t orow = ((b * a.heads + h) * a.len + l) * kD + j * kPer;
-  store_row8<QT>(a.q_out, orow, q);
-  store_row8<KT>(a.k_out, orow, k);
+  const int64_t orow = (b * a.heads + h) * a.len + l;
+  store_row8<QT>(a.q_out, orow, j, q);
+  store_row8<KT>(a.k_out, orow, j, k);
   // v keeps the projection's values and type (the bias, when given, added in
   // fp32 and rounded to that type once)
   if (a.v_bias != nullptr) {
     add_bias(v, a.v_bias + bias_off);
-    store_row8<IT>(a.v_out, orow, v);
+    store_row8<IT>(a.v_out, orow, j, v);
   } else {
-    store_raw8<IT>(a.v_out, orow, rv);
+    store_raw8<IT>(a.v_out, orow, j, rv);
   }
 
   if (a.append_offsets != nullptr) {
     const int32_t off = a.append_offsets[h];
     if (off >= 0 && static_cast<int64_t>(off) + l < a.slab_capacity) {
-      const int64_t srow = (b * a.slab_capacity + off + l) * kD + j * kPer;
-      store_row8<KT>(a.slab_k, srow, k);
-      if (a.v_bias != nullptr) store_row8<IT>(a.slab_v, srow, v);
-      else store_raw8<IT>(a.slab_v, srow, rv);
+      const int64_t srow = b * a.slab_capacity + off + l;
+      store_row8<KT>(a.slab_k, srow, j, k);
+      if (a.v_bias != nullptr) store_row8<IT>(a.slab_v, srow, j, v);
+      else store_raw8<IT>(a.slab_v, srow, j, rv);
     }
   }
 }
@@ -266,8 +301,9 @@ hipError_t launch_for_input(const ProduceArgs& a, dim3 grid, hipStream_t stream)
 
 hipError_t launch_produce(const ProduceArgs& a, hipStream_t stream) {
   if (a.rows <= 0) return hipSuccess;
+  // 32-bit row numbers: 2^31 rows would be 1.6 TB of 16-bit outputs
+  if (a.rows > 0x7fffffffLL - kRowsPerBlock) return hipErrorInvalidConfiguration;
   const int64_t blocks = (a.rows + kRowsPerBlock - 1) / kRowsPerBlock;
-  if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   const dim3 grid(static_cast<uint32_t>(blocks));
   switch (a.qkv_dtype) {
     case kBF16: return launch_for_input<kBF16>(a, grid, stream);

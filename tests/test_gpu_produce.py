@@ -82,6 +82,33 @@ def test_producer_against_oracle(device, scale_ind, B, H):
     assert np.array_equal(to_np(v.float()), wv)
 
 
+@pytest.mark.parametrize("L,H", [(1, 1), (1, 5), (15, 3), (17, 16), (33, 7)])
+@pytest.mark.parametrize("proj", [torch.bfloat16, torch.float32])
+def test_producer_row_groups(device, L, H, proj):
+    """Workgroups of 16 rows that end inside a token, a batch row or the launch,
+    with the append: outputs against the oracle, v and slab rows bit for bit."""
+    B = 3
+    print(f"[produce] row groups L {L} H {H} {proj}", flush=True)
+    qkv = (_qkv(B, L, H, 60 + L).float() * 1.0009765625).to(proj)
+    sm = _scale_mul(H, 61)
+    table = P.rope2d_freqs_table(D, [(1, 6, 6)], 2, 36)
+    offsets = [-1 if h % 3 == 1 else 2 + h * L for h in range(H)]
+    cap = 3 + H * L
+    slab = (torch.zeros((B, cap, D), device=device), torch.zeros((B, cap, D), device=device, dtype=proj))
+    q, k, v = P.qkv_produce(qkv.to(device), H, scale_mul=sm.to(device), rope_table=table.to(device),
+                            append=(*slab, torch.tensor(offsets, dtype=torch.int32, device=device)))
+    torch.cuda.synchronize(device)
+    wq, wk, wv = O.produce(qkv.float().numpy().reshape(B, L, 3, H, D), scale_mul=sm.numpy(), table=table.numpy(),
+                           start=0)
+    _check_qk(q, k, wq, wk, sm, H)
+    assert np.array_equal(to_np(v.float()), wv)
+    want = [torch.zeros_like(t) for t in slab]
+    for h, off in enumerate(offsets):
+        if off >= 0:
+            want[0][:, off:off + L], want[1][:, off:off + L] = k[:, h], v[:, h]
+    assert torch.equal(slab[0], want[0]) and torch.equal(slab[1], want[1])
+
+
 def test_producer_bias_no_normalize_and_bf16_out(device):
     B, L, H = 2, 576, 16
     qkv = _qkv(B, L, H, 3)
