@@ -133,11 +133,11 @@ struct SplitOperands {
   const int32_t* seg_counts;
   int64_t slab_capacity;
   int64_t cur_rows;     // batch * heads * cur_len
-  int64_t slab_blocks;  // set by the launch
+  int64_t slab_blocks;  // set by the launch, as slab_chunks
+  int64_t slab_chunks;
   int32_t batch;
   int32_t heads;
   int32_t max_segments;
-  int32_t slab_chunks;  // set by the launch
 };
 hipError_t launch_split_operands(SplitOperands o, bool with_v, hipStream_t stream);
 // The append of AttnArgs::append_offsets as a launch of its own.

@@ -115,13 +115,8 @@ __device__ __forceinline__ void exp_half(f32x16_t& s, float m_run, float c, floa
   l_run += p0 + p1;
 }
 
-// fp32 rows -> split rows: 16 threads per row, 8 values each.
-__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ src, uint8_t* __restrict__ dst,
-                                                         int64_t rows) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  const int64_t row = i >> 4;
-  if (row >= rows) return;
-  const int c = static_cast<int>(i & 15);
+// fp32 row -> split row: 16 threads per row, 8 values each (thread c of the row).
+__device__ __forceinline__ void split_row(const float* src, uint8_t* dst, int64_t row, int c) {
   const f32x4_t x = *reinterpret_cast<const f32x4_t*>(src + row * kD + c * 8);
   const f32x4_t y = *reinterpret_cast<const f32x4_t*>(src + row * kD + c * 8 + 4);
   const float v[8] = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
@@ -138,83 +133,64 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
   *reinterpret_cast<u32x4_t*>(out + kD * 2 + c * 16) = lo;
 }
 
-// What an attention call on fp32 K (and V) rows splits before it: the current
-// rows, and of the slab only the rows that the tables' segments hold, K and V
-// (blockIdx.y) in one launch.  A block moves 64 rows at a time, 16 threads per
-// row, 4 rows' loads in flight per thread.  A head's retained rows are one
-// stream (its segments back to back) that slab_chunks blocks share, and the
-// slab's blocks come first: they wait for the tables, and one long head must
-// not end the launch late (2304 tokens, 16 heads, B = 2, K and V, 75 MB in and
-// 75 MB out: 34 us, against 110 us with one block per head).
-constexpr int kSplitBlockRows = 64;
-constexpr int64_t kSplitSlabBlocks = 512;  // about as many for the slab: most find few rows or none
-
-__device__ __forceinline__ void split_row_group(const float* src, uint8_t* dst, const int64_t (&rows)[4]) {
-  const int c = threadIdx.x & 15;
-  f32x4_t x[4], y[4];
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    if (rows[u] < 0) continue;
-    x[u] = *reinterpret_cast<const f32x4_t*>(src + rows[u] * kD + c * 8);
-    y[u] = *reinterpret_cast<const f32x4_t*>(src + rows[u] * kD + c * 8 + 4);
-  }
-#pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    if (rows[u] < 0) continue;
-    const float v[8] = {x[u][0], x[u][1], x[u][2], x[u][3], y[u][0], y[u][1], y[u][2], y[u][3]};
-    u32x4_t hi, lo;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      hi[k] = pack2<kBF16>(v[2 * k], v[2 * k + 1]);
-      const float h0 = __builtin_bit_cast(float, hi[k] << 16);
-      const float h1 = __builtin_bit_cast(float, hi[k] & 0xffff0000u);
-      lo[k] = pack2<kBF16>(v[2 * k] - h0, v[2 * k + 1] - h1);
-    }
-    uint8_t* const out = dst + rows[u] * kSRowBytes;
-    *reinterpret_cast<u32x4_t*>(out + c * 16) = hi;
-    *reinterpret_cast<u32x4_t*>(out + kD * 2 + c * 16) = lo;
-  }
+__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ src, uint8_t* __restrict__ dst,
+                                                         int64_t rows) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >> 4 < rows) split_row(src, dst, i >> 4, static_cast<int>(i & 15));
 }
 
+// What an attention call on fp32 K (and V) rows splits before it: the current
+// rows, and of the slab only the rows that the tables' segments hold, K and V
+// (blockIdx.y) in one launch.  HBM bound.  A block of current rows moves 16, one
+// per 16 threads: short blocks, many in flight.  A block of the slab owns 32
+// consecutive rows of it: its threads mark in one word of LDS which of them any
+// head's segment holds (one round trip for the tables, all entries at once) and
+// move those; every block does about the same, however the rows are spread over
+// the heads.  The slab's blocks come first, as they wait for the tables.  Whole
+// calls, B=2, 16 heads: 2272 tokens, fp32 q/k, heads of very different retained
+// lengths 224.8 -> 215.5 us against each head's rows walked as one stream by 16
+// blocks of 64-row steps (216.5 with every slab row split, in two launches);
+// 2304 tokens all fp32, a tenth retained 323 -> 318 us.  Non-temporal stores
+// cost 1 to 3 % of a call: the attention reads the rows next.
+constexpr int kSplitCurRows = 16;
+constexpr int kSplitSlabRows = 32;
+
 __global__ __launch_bounds__(256) void split_operands_kernel(const SplitOperands o) {
-  __shared__ int32_t seg_start[kMaxSegments];
-  __shared__ int32_t seg_pref[kMaxSegments + 1];
+  __shared__ uint32_t live;
   const bool is_v = blockIdx.y != 0;
-  const int sub = threadIdx.x >> 4;
+  const int tid = threadIdx.x;
+  const int sub = tid >> 4, c = tid & 15;
   const int64_t blk = blockIdx.x;
-  int64_t rows[4];
   if (blk >= o.slab_blocks) {
-    const int64_t r0 = (blk - o.slab_blocks) * kSplitBlockRows;
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int64_t r = r0 + sub + 16 * u;
-      rows[u] = r < o.cur_rows ? r : -1;
-    }
-    split_row_group(is_v ? o.cur_v : o.cur_k, is_v ? o.cur_v_out : o.cur_k_out, rows);
+    const int64_t row = (blk - o.slab_blocks) * kSplitCurRows + sub;
+    if (row < o.cur_rows) split_row(is_v ? o.cur_v : o.cur_k, is_v ? o.cur_v_out : o.cur_k_out, row, c);
     return;
   }
-  const int32_t bh = static_cast<int32_t>(blk / o.slab_chunks);
-  const int32_t chunk = static_cast<int32_t>(blk - static_cast<int64_t>(bh) * o.slab_chunks);
-  WorkItem w;
-  w.b = bh / o.heads;
-  w.h = bh - w.b * o.heads;
-  load_head_segments<256>(o.seg_starts, o.seg_ends, o.seg_counts, o.slab_capacity, o.max_segments, w, seg_start,
-                          seg_pref);
-  const float* const src = (is_v ? o.slab_v : o.slab_k) + w.b * o.slab_capacity * kD;
-  uint8_t* const dst = (is_v ? o.slab_v_out : o.slab_k_out) + w.b * o.slab_capacity * kSRowBytes;
-  int s = 0;  // positions grow, so the segment search walks forward
-  for (int32_t p0 = chunk * kSplitBlockRows; p0 < w.R; p0 += o.slab_chunks * kSplitBlockRows) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int32_t p = p0 + sub + 16 * u;
-      rows[u] = -1;
-      if (p < w.R) {
-        while (seg_pref[s + 1] <= p) ++s;
-        rows[u] = seg_start[s] + (p - seg_pref[s]);
-      }
-    }
-    split_row_group(src, dst, rows);
+  const int64_t cap = o.slab_capacity;
+  const int64_t b = blk / o.slab_chunks;
+  const int64_t r0 = (blk - b * o.slab_chunks) * kSplitSlabRows;
+  if (tid == 0) live = 0;
+  __syncthreads();
+  uint32_t mine = 0;
+  for (int32_t e = tid; e < o.heads * o.max_segments; e += 256) {
+    const int32_t h = e / o.max_segments;
+    // rows [st, en) of the entry, clamped to the slab as the attention clamps them
+    int64_t st = o.seg_starts[e], en = o.seg_ends[e];
+    if (e - h * o.max_segments >= o.seg_counts[h]) continue;
+    st = (st < 0 ? 0 : st) - r0;
+    en = (en > cap ? cap : en) - r0;
+    st = st < 0 ? 0 : st;
+    en = en > kSplitSlabRows ? kSplitSlabRows : en;
+    if (en > st) mine |= static_cast<uint32_t>(((1ull << (en - st)) - 1) << st);
   }
+  if (mine != 0) atomicOr(&live, mine);
+  __syncthreads();
+  const uint32_t rows = live;
+  const float* const src = is_v ? o.slab_v : o.slab_k;
+  uint8_t* const dst = is_v ? o.slab_v_out : o.slab_k_out;
+#pragma unroll
+  for (int u = 0; u < kSplitSlabRows / 16; ++u)
+    if ((rows >> (sub + 16 * u)) & 1) split_row(src, dst, b * cap + r0 + sub + 16 * u, c);
 }
 
 template <int VDT>
@@ -977,12 +953,9 @@ hipError_t launch_attention_split(const AttnArgs& a, const attn::Scalars& s, hip
 }
 
 hipError_t launch_split_operands(SplitOperands o, bool with_v, hipStream_t stream) {
-  const int64_t cur_blocks = (o.cur_rows + kSplitBlockRows - 1) / kSplitBlockRows;
-  const int64_t bh = static_cast<int64_t>(o.batch) * o.heads;
-  const int64_t share = kSplitSlabBlocks / bh < 4 ? 4 : kSplitSlabBlocks / bh;
-  const int64_t chunks = (o.slab_capacity + kSplitBlockRows - 1) / kSplitBlockRows;
-  o.slab_chunks = static_cast<int32_t>(chunks < share ? chunks : share);
-  o.slab_blocks = o.max_segments > 0 ? bh * o.slab_chunks : 0;
+  const int64_t cur_blocks = (o.cur_rows + kSplitCurRows - 1) / kSplitCurRows;
+  o.slab_chunks = o.max_segments > 0 ? (o.slab_capacity + kSplitSlabRows - 1) / kSplitSlabRows : 0;
+  o.slab_blocks = o.batch * o.slab_chunks;
   const int64_t blocks = cur_blocks + o.slab_blocks;
   if (blocks <= 0) return hipSuccess;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;
