@@ -138,8 +138,35 @@ def load():
                 f"{LIB_PATH} reports ABI version {have >> 16}.{(have >> 8) & 255}.{have & 255}; these "
                 f"bindings need {ABI_VERSION >> 16}.{(ABI_VERSION >> 8) & 255}.{ABI_VERSION & 255} -- rebuild it "
                 "with `python heatkv_amd/csrc/build.py`")
+        _load_op_call(lib)
         _lib = lib
     return _lib
+
+
+# The native call path of the operators (csrc/op_call.cpp), set by load().
+op_call = None
+_OP_KNOBS = ("REAL_PRUNING_FUSED_QK_DOT_MODE", "REAL_PRUNING_FUSED_VALUE_DOT_MODE", "HKV_ATTN_SPLIT",
+             "HKV_ATTN_SPLIT_ROWS")
+
+
+def _load_op_call(lib) -> None:
+    """Imports the extension and gives it the library's entry points and the
+    dicts it looks into: the environment (with any of ``_OP_KNOBS`` set, calls
+    take the operators' Python bodies), the per-stream workspaces and the
+    checked devices."""
+    global op_call
+    try:
+        from . import _op_call
+    except ImportError as e:
+        raise RuntimeError(f"the native call path heatkv_amd/_op_call.so cannot be loaded ({e}); build it with "
+                           "`python heatkv_amd/csrc/build.py`") from e
+    if not isinstance(_ENV_DATA, dict):  # pragma: no cover - another platform's os.environ
+        return
+    names = ("hkv_segmented_attention", "hkv_segmented_attention_split", "hkv_segmented_attention_split_bytes",
+             "hkv_segmented_attention_item_shape", "hkv_qkv_produce", "hkv_pack_segments")
+    _op_call.init(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), _ENV_DATA,
+                  tuple(os.environ.encodekey(n) for n in _OP_KNOBS), _workspaces, _device_ok)
+    op_call = _op_call
 
 
 def last_error() -> str:

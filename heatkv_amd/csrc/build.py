@@ -1,8 +1,10 @@
-"""Build libheatkv.so (gfx950) in-tree from the HIP sources in this directory.
+"""Build libheatkv.so (gfx950) in-tree from the HIP sources in this directory,
+and the Python extension ``_op_call`` (host C++ only) beside it.
 
 Usage: ``python heatkv_amd/csrc/build.py`` or ``heatkv_amd.csrc.build.build()``.
 Each source compiles to an object in ``_build/`` in parallel, then one link
-writes ``heatkv_amd/libheatkv.so``.  Always recompiles (it is the build check).
+writes ``heatkv_amd/libheatkv.so``; ``op_call.cpp`` compiles meanwhile to
+``heatkv_amd/_op_call.so``.  Always recompiles (it is the build check).
 """
 
 from __future__ import annotations
@@ -44,6 +46,27 @@ EXTRA = {
 }
 
 
+OP_CALL = os.path.join(PKG, "_op_call.so")
+
+
+def _op_call_command(out):
+    """The extension's compile and link: torch's headers and libraries of the
+    running interpreter (already loaded when the package imports it)."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{os.path.join(ROOT, 'include')}",
+            "-isystem", os.path.join(root, "include"),
+            "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),
+            "-isystem", os.path.join(rocm, "include"), "-isystem", sysconfig.get_paths()["include"],
+            os.path.join(HERE, "op_call.cpp"), "-o", out, f"-L{os.path.join(root, 'lib')}",
+            "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python"]
+
+
 def _hipcc():
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     cand = os.path.join(rocm, "bin", "hipcc")
@@ -69,6 +92,7 @@ def build(verbose: bool = False) -> str:
         obj = os.path.join(out_dir, src.replace(".hip", ".o"))
         objs.append(obj)
         cmds.append([hipcc, *FLAGS, *EXTRA.get(src, []), "-c", os.path.join(HERE, src), "-o", obj])
+    cmds.append(_op_call_command(OP_CALL + ".tmp"))
     with ThreadPoolExecutor(max_workers=len(cmds)) as ex:
         for msg in ex.map(_run, cmds):
             if verbose and msg.strip():
@@ -76,6 +100,7 @@ def build(verbose: bool = False) -> str:
     tmp = LIB + ".tmp"
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objs, "-o", tmp])
     os.replace(tmp, LIB)
+    os.replace(OP_CALL + ".tmp", OP_CALL)
     return LIB
 
 

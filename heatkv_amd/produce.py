@@ -187,6 +187,12 @@ def qkv_produce(
     valid), the K format the attention's split-row kernel reads: calls with
     ``k_split_rows=True`` then skip their own split.
     """
+    native = _lib.op_call
+    if native is not None and q_bias is None and v_bias is None:
+        out = native.produce(qkv, num_heads, scale_mul, rope_table, rope_start_row, normalize, eps, qk_dtype, append,
+                             k_split_rows)
+        if out is not None:
+            return out
     if not qkv.is_cuda:
         raise RuntimeError("qkv_produce runs on the GPU only (HIP kernel); got a CPU tensor")
     if qkv.dtype not in (torch.bfloat16, torch.float16, torch.float32):

@@ -319,6 +319,10 @@ def pack_flat_segments_kv(
     ``hkv_pack_segments``.  ``_bind`` (internal): a list that receives what
     :class:`BoundPack` needs to repeat this launch.
     """
+    native = _lib.op_call
+    if (native is not None and _bind is None
+            and native.pack(dst_k, dst_v, src_k, src_v, dst_starts, src_starts, lengths, max_length, block_t)):
+        return dst_k, dst_v
     for name, tensor in (("dst_k", dst_k), ("dst_v", dst_v), ("src_k", src_k), ("src_v", src_v)):
         if tensor.ndim != 3:
             raise ValueError(f"pack_flat_segments_kv expects {name} shaped [B, S, D]")
@@ -452,6 +456,13 @@ def fused_real_pruning_flat_segmented_attention(
     (real_pruning_fused_attention.py:445-591); the work is the HIP kernel
     ``hkv_segmented_attention``.
     """
+    native = _lib.op_call
+    if native is not None and append_offsets is None and append_also is None and _bind is None:
+        out = native.attention(q, persisted_k, persisted_v, segment_starts, segment_ends, segment_counts, current_k,
+                               current_v, softmax_scale, softmax_mode, return_lse, out_dtype, work_plan, k_split_rows,
+                               _SPLIT_VALUES_ROWS)
+        if out is not None:
+            return out
     if q.ndim != 4 or current_k.ndim != 4 or current_v.ndim != 4:
         raise ValueError("q, current_k, and current_v must have shape [B, H, L, D]")
     if q.shape != current_k.shape or q.shape != current_v.shape:
