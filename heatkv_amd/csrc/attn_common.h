@@ -549,13 +549,15 @@ __device__ __forceinline__ int32_t xcd_item(int32_t j, int32_t groups, int32_t n
 template <int ROW_BYTES = 1>
 __device__ __forceinline__ void fill_rowtab(int tile, int32_t* rowtab, int& cur_seg, int nseg, int R,
                                             const int32_t* seg_start, const int32_t* seg_pref,
-                                            int32_t past_end = -1) {
+                                            int32_t past_end = -1, int before = 0) {
   const int lane = threadIdx.x & 63;
-  const int j0 = tile * kBN;
+  const int j0 = tile * kBN - before;
   while (cur_seg < nseg && seg_pref[cur_seg + 1] <= j0) ++cur_seg;
   const int j = j0 + lane;
+// `before` > 0: the tile starts that many positions ahead of tile * 64, and
+// positions below 0 (a mixed tile's current rows) get `past_end` too.
   int32_t row = past_end;
-  if (j < R) {
+  if (j >= 0 && j < R) {
     int s = cur_seg;
     while (seg_pref[s + 1] <= j) ++s;
     row = (seg_start[s] + (j - seg_pref[s])) * ROW_BYTES;

@@ -92,7 +92,22 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 // SIMD being in the opposite phase.  Same ring (K half of stage t % 2 holds
 // K(t), V half holds V(t)), same row tables (3 slots, filled 3 tiles ahead),
 // one barrier per tile, one tile of DMA in flight per wave.
-template <int QDT, int KDT, int VDT>
+//
+// MIXED: the last tile of the current scale is partial (L % 64 rows) and the
+// first prior rows fill it, so the key stream is L + R rows without a gap: tile
+// t holds stream rows [64 t, 64 t + 64).  In that one tile (`nfull`) each DMA
+// instruction is issued twice, for the lanes of current rows and for the lanes
+// of prior rows (lanes that are off leave their 16 bytes of LDS alone).  Worth a tile per item where the two remainders fit one: an
+// early scale of 16 or 36 tokens with its 5 or 21 kept rows is one tile instead
+// of two.  B=2, 16 heads, a tenth retained, planned, us, off / on: 4 tokens 7.6 /
+// 6.6, 16: 7.9 / 6.7, 36: 8.3 / 7.3, 144: 11.4 / 10.1, 400: 18.2 / 17.0; not
+// planned 9.0 / 7.7, 9.1 / 8.1, 9.4 / 8.4, 12.1 / 11.0, 18.9 / 18.0.  From about
+// 1000 tokens one tile in twenty no longer pays for the lanes' tests in the loop
+// (1023 tokens 41.0 / 41.8 planned, 4087 tokens 336 / 341 not planned): off from
+// kMixedBelow, and at multiples of 64, which have no such tile.
+constexpr int32_t kMixedBelow = 10 * kBN;  // current rows
+
+template <int QDT, int KDT, int VDT, bool MIXED>
 __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
     const int32_t* __restrict__ plan_p, const int32_t n_units, const AttnArgs a, const Scalars sc,
     const int32_t n_qt, const RoundSplit split) {
@@ -141,10 +156,13 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
   Unit un;
   WorkItem w;
   int32_t t_begin, t_end, parts;
-  const int32_t ntc = (L + kBN - 1) / kBN;
   // An item's key stream: its ntc current-scale tiles first (addressed
-  // without any table), then its R retained prior rows, ntp tiles through the
-  // row tables.
+  // without any table), then its R retained prior rows through the row tables;
+  // tiles from nfull on hold prior rows (MIXED: nfull the current rows' rest,
+  // `rest` of them, before them).
+  const int32_t ntc = (L + kBN - 1) / kBN;
+  const int32_t nfull = MIXED ? L / kBN : ntc;
+  const int32_t rest = MIXED ? L - nfull * kBN : 0;
   int32_t p0 = 0, p1 = 0;
   bool cut = false;
   bool shared = false;  // alternate the wave priority by tile (the plan says so)
@@ -204,29 +222,41 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
   const int32_t off0 = key0 * (kD * 2) + col0;
   const uint32_t ring_lds = lds_address(ring) + wave * kDmaPerWave * 1024;
 
-  // This wave's tensor (K or V) of current-scale tile c into stage c % 2.
+  // This wave's tensor (K or V) of current-scale tile c into stage c % 2; of
+  // the mixed tile the lanes of current rows.
   auto issue_cur = [&](int c) {
     const uint32_t dst = ring_lds + (c % NS) * kStageBytes;
     const uint32_t skip = static_cast<uint32_t>(c) * (kBN * kD * 2);
     const u32x4_t d_cur = make_desc(cur_base + skip, cur_bytes - skip);
+    const int lim = MIXED && c == nfull ? rest : kBN;
     if (k_wave) {
-      dma16_at<0>(d_cur, dst, off0);
-      dma16_at<32>(d_cur, dst + 1024, off0);
-      dma16_at<64>(d_cur, dst + 2048, off0);
-      dma16_at<96>(d_cur, dst + 3072, off0);
-      dma16_at<128>(d_cur, dst + 4096, off0);
-      dma16_at<160>(d_cur, dst + 5120, off0);
-      dma16_at<192>(d_cur, dst + 6144, off0);
-      dma16_at<224>(d_cur, dst + 7168, off0);
+      if (!MIXED || key0 < lim) {
+        dma16_at<0>(d_cur, dst, off0);
+        dma16_at<32>(d_cur, dst + 1024, off0);
+        dma16_at<64>(d_cur, dst + 2048, off0);
+        dma16_at<96>(d_cur, dst + 3072, off0);
+        dma16_at<128>(d_cur, dst + 4096, off0);
+        dma16_at<160>(d_cur, dst + 5120, off0);
+        dma16_at<192>(d_cur, dst + 6144, off0);
+        dma16_at<224>(d_cur, dst + 7168, off0);
+      }
     } else {
-      dma16_at<0>(d_cur, dst, off0);
-      dma16_at<128>(d_cur, dst + 1024, off0);
-      dma16_at<2048>(d_cur, dst + 2048, off0);
-      dma16_at<2176>(d_cur, dst + 3072, off0);
-      dma16_at<4096>(d_cur, dst + 4096, off0);
-      dma16_at<4224>(d_cur, dst + 5120, off0);
-      dma16_at<6144>(d_cur, dst + 6144, off0);
-      dma16_at<6272>(d_cur, dst + 7168, off0);
+      if (!MIXED || key0 < lim) {
+        dma16_at<0>(d_cur, dst, off0);
+        dma16_at<128>(d_cur, dst + 1024, off0);
+      }
+      if (!MIXED || key0 + 8 < lim) {
+        dma16_at<2048>(d_cur, dst + 2048, off0);
+        dma16_at<2176>(d_cur, dst + 3072, off0);
+      }
+      if (!MIXED || key0 + 16 < lim) {
+        dma16_at<4096>(d_cur, dst + 4096, off0);
+        dma16_at<4224>(d_cur, dst + 5120, off0);
+      }
+      if (!MIXED || key0 + 24 < lim) {
+        dma16_at<6144>(d_cur, dst + 6144, off0);
+        dma16_at<6272>(d_cur, dst + 7168, off0);
+      }
     }
   };
   // A planned unit whose first tile is a current-scale one (every whole item,
@@ -250,7 +280,7 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
   if (planned) {
     load_head_segments<kThreads>(a.seg_starts, a.seg_ends, a.seg_counts, cap, a.max_segments, w, seg_start,
                                  seg_pref);
-    const int32_t ntiles = (w.R + kBN - 1) / kBN + ntc;
+    const int32_t ntiles = MIXED ? (w.R + L + kBN - 1) / kBN : (w.R + kBN - 1) / kBN + ntc;
     t_begin = p0 < 0 ? 0 : (p0 > ntiles ? ntiles : p0);
     t_end = p1 < t_begin ? t_begin : (p1 > ntiles ? ntiles : p1);
     if (!cut) {  // a whole item, whatever the plan's range says
@@ -284,48 +314,66 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
     return;
   }
 
-  // This wave's tensor (K or V) of tile `tile` into stage tile % 2.
-  auto issue_tile = [&](int tile) {
-    if (tile < ntc) {
-      issue_cur(tile);
-      return;
-    }
-    const int p = tile - ntc;
+  // ... of tile `tile` >= nfull, its prior rows; of the mixed tile the other
+  // lanes (zeros past the stream's end).
+  auto issue_prior = [&](int tile) {
+    const int p = tile - nfull;
     const uint32_t dst = ring_lds + (tile % NS) * kStageBytes;
     const int32_t* rt = rowtab[p % 3];
+    const int from = MIXED && p == 0 ? rest : 0;
     if (k_wave) {
-      const int32_t r = rt[key0] + col0;
-      dma16_at<0>(d_prior, dst, r);
-      dma16_at<32>(d_prior, dst + 1024, r);
-      dma16_at<64>(d_prior, dst + 2048, r);
-      dma16_at<96>(d_prior, dst + 3072, r);
-      dma16_at<128>(d_prior, dst + 4096, r);
-      dma16_at<160>(d_prior, dst + 5120, r);
-      dma16_at<192>(d_prior, dst + 6144, r);
-      dma16_at<224>(d_prior, dst + 7168, r);
+      if (!MIXED || key0 >= from) {
+        const int32_t r = rt[key0] + col0;
+        dma16_at<0>(d_prior, dst, r);
+        dma16_at<32>(d_prior, dst + 1024, r);
+        dma16_at<64>(d_prior, dst + 2048, r);
+        dma16_at<96>(d_prior, dst + 3072, r);
+        dma16_at<128>(d_prior, dst + 4096, r);
+        dma16_at<160>(d_prior, dst + 5120, r);
+        dma16_at<192>(d_prior, dst + 6144, r);
+        dma16_at<224>(d_prior, dst + 7168, r);
+      }
     } else {
       const int32_t r0 = rt[key0] + col0, r1 = rt[key0 + 8] + col0;
       const int32_t r2 = rt[key0 + 16] + col0, r3 = rt[key0 + 24] + col0;
-      dma16_at<0>(d_prior, dst, r0);
-      dma16_at<128>(d_prior, dst + 1024, r0);
-      dma16_at<0>(d_prior, dst + 2048, r1);
-      dma16_at<128>(d_prior, dst + 3072, r1);
-      dma16_at<0>(d_prior, dst + 4096, r2);
-      dma16_at<128>(d_prior, dst + 5120, r2);
-      dma16_at<0>(d_prior, dst + 6144, r3);
-      dma16_at<128>(d_prior, dst + 7168, r3);
+      if (!MIXED || key0 >= from) {
+        dma16_at<0>(d_prior, dst, r0);
+        dma16_at<128>(d_prior, dst + 1024, r0);
+      }
+      if (!MIXED || key0 + 8 >= from) {
+        dma16_at<0>(d_prior, dst + 2048, r1);
+        dma16_at<128>(d_prior, dst + 3072, r1);
+      }
+      if (!MIXED || key0 + 16 >= from) {
+        dma16_at<0>(d_prior, dst + 4096, r2);
+        dma16_at<128>(d_prior, dst + 5120, r2);
+      }
+      if (!MIXED || key0 + 24 >= from) {
+        dma16_at<0>(d_prior, dst + 6144, r3);
+        dma16_at<128>(d_prior, dst + 7168, r3);
+      }
     }
   };
-  auto valid_of = [&](int t) { return t < ntc ? min(kBN, L - t * kBN) : min(kBN, R - (t - ntc) * kBN); };
+  // This wave's tensor (K or V) of tile `tile` into stage tile % 2.
+  auto issue_tile = [&](int tile) {
+    if (MIXED ? tile <= nfull : tile < nfull) issue_cur(tile);
+    if (tile >= nfull) issue_prior(tile);
+  };
+  auto valid_of = [&](int t) {
+    if constexpr (MIXED) return min(kBN, L + R - t * kBN);
+    return t < ntc ? min(kBN, L - t * kBN) : min(kBN, R - (t - ntc) * kBN);
+  };
 
   int cur_seg = 0;
   if (wave == 0) {
     for (int t = t_begin; t < t_begin + 3 && t < t_end; ++t)
-      if (t >= ntc)
-        fill_rowtab<kD * 2>(t - ntc, rowtab[(t - ntc) % 3], cur_seg, w.nseg, R, seg_start, seg_pref, kPastEnd);
+      if (t >= nfull)
+        fill_rowtab<kD * 2>(t - nfull, rowtab[(t - nfull) % 3], cur_seg, w.nseg, R, seg_start, seg_pref, kPastEnd,
+                            rest);
   }
   __syncthreads();
   if (!early) issue_tile(t_begin);
+  else if (MIXED && t_begin == nfull) issue_prior(t_begin);
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) qf[ks] ^= sc.q_sign;
 
@@ -400,9 +448,9 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
     } else {
       if (t + 1 < t_end) issue_tile(t + 1);
     }
-    if (wave == 0 && t + 3 < t_end && t + 3 >= ntc)
-      fill_rowtab<kD * 2>(t + 3 - ntc, rowtab[(t + 3 - ntc) % 3], cur_seg, w.nseg, R, seg_start, seg_pref,
-                          kPastEnd);
+    if (wave == 0 && t + 3 < t_end && t + 3 >= nfull)
+      fill_rowtab<kD * 2>(t + 3 - nfull, rowtab[(t + 3 - nfull) % 3], cur_seg, w.nseg, R, seg_start, seg_pref,
+                          kPastEnd, rest);
     u32x4_t pf[4];
     qk(snext, t + 1);
     exp_tile(scur, m_run, sc.c, l_run);
@@ -505,8 +553,12 @@ hipError_t launch(const AttnArgs& a, const Scalars& s, hipStream_t st) {
   if (blocks + copies <= 0) return hipSuccess;
   if (blocks + copies > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   b.append_first = static_cast<int32_t>(blocks);
-  seg_attn_pipe_kernel<DT, DT, VDT><<<dim3(static_cast<uint32_t>(blocks + copies)), 256, 0, st>>>(
-      b.plan, b.plan != nullptr ? static_cast<int32_t>(blocks) : 0, b, s, n_qt, split);
+  const dim3 grid(static_cast<uint32_t>(blocks + copies));
+  const int32_t units = b.plan != nullptr ? static_cast<int32_t>(blocks) : 0;
+  if (a.cur_len % kBN != 0 && a.cur_len < kMixedBelow)
+    seg_attn_pipe_kernel<DT, DT, VDT, true><<<grid, 256, 0, st>>>(b.plan, units, b, s, n_qt, split);
+  else
+    seg_attn_pipe_kernel<DT, DT, VDT, false><<<grid, 256, 0, st>>>(b.plan, units, b, s, n_qt, split);
   return hipGetLastError();
 }
 
