@@ -445,32 +445,40 @@ __device__ __forceinline__ WorkItem plan_work(const int32_t* __restrict__ seg_st
 // a slot model gives 116 us against 133 us for cutting the lightest).  With
 // N <= G, the first min(N, G - N) are cut, so the one round is not set by
 // the heaviest item.  N >= 2G launches are not cut.  An item with fewer than
-// 2 kMinPartTiles key tiles still runs whole: its second part finds too few
+// 2 min_part key tiles still runs whole: its second part finds too few
 // tiles and leaves at once.  A part leaves its partial result (unnormalized
 // O, running max and sum) in a workspace record; the part that completes an
 // item last merges both records in part order.  Workgroup ids: with
 // whole_first, items [two, N) whole, then the cut items' parts; otherwise
 // the cut items' parts, then items [two, N) whole.  The parts of a cut item
-// are adjacent when every item has at least 2 kMinPartTiles tiles;
+// are adjacent when every item has at least 2 min_part tiles;
 // otherwise all first parts come before all second parts: workgroup ids are
 // dealt to the 8 XCDs round robin, and adjacent second parts that leave at
 // once would leave half of the XCDs idle.  (Measured on the 2B scales:
 // adjacent parts run scale 9 in 36 us against 40 us grouped; grouped parts
 // run scale 8 in 21 us against 30 us adjacent.)
-// Key tiles a part of a cut item must have at least (measured on the 2B
-// scales: parts of ~8.5 tiles gain 13 %, parts of ~5 tiles lose 20 %).
-constexpr int32_t kMinPartTiles = 8;
+// Key tiles a part of a cut item must have at least (min_part): 5, or 4 where
+// every part has a CU to itself (a quarter of the slots).  16 heads, not
+// planned, us at 8 / 5 / 4 tiles: 576 tokens, B=2 25.8 / 22.1 / 23.9 (fp32 q/k
+// 37 / 31.6 / 33.5), B=1 24.1 / 19.4 / 19.9; 400 tokens, heads of uneven lengths,
+// B=2 25.4 / 20.3 / 20.5 (38.6 / 28.6 / 29.6); 256 tokens, the same, 17.2 / 17.1 /
+// 15.3 (24.7 / 24.8 / 20.6), but 128 items of 256 parts, B=4, 32 heads 21.4 / 21.3 /
+// 22.4.
+constexpr int32_t kMinPartTiles = 5;
+constexpr int32_t kMinPartTilesAlone = 4;
 
 struct RoundSplit {
   int32_t items;        // N
   int32_t two;          // cut items: [0, two) in longest-first order
   int32_t grouped;      // first parts, then second parts (else each item's two parts adjacent)
   int32_t whole_first;  // whole items before the cut items' parts
+  int32_t min_part;     // key tiles of a part at least
 };
 
 // `min_tiles`: key tiles every item has at least (its current-scale tiles).
 __host__ __device__ __forceinline__ RoundSplit round_split(int32_t items, int32_t slots, int32_t min_tiles) {
-  RoundSplit t{items, 0, min_tiles < 2 * kMinPartTiles ? 1 : 0, 0};
+  const int32_t min_part = 4LL * items <= slots ? kMinPartTilesAlone : kMinPartTiles;
+  RoundSplit t{items, 0, min_tiles < 2 * min_part ? 1 : 0, 0, min_part};
   if (slots <= 0 || items >= 2 * slots) return t;
   if (items > slots) {
     t.two = 2 * slots - items;
@@ -546,6 +554,8 @@ __device__ __forceinline__ int32_t xcd_item(int32_t j, int32_t groups, int32_t n
 // stream position -> slab row * ROW_BYTES, or `past_end` past R.  With
 // ROW_BYTES = 1 the entries are row indices.  `cur_seg` walks forward with
 // the tiles (callers fill tiles in increasing order).
+// `before` > 0: the tile starts that many positions ahead of tile * 64, and
+// positions below 0 (a mixed tile's current rows) get `past_end` too.
 template <int ROW_BYTES = 1>
 __device__ __forceinline__ void fill_rowtab(int tile, int32_t* rowtab, int& cur_seg, int nseg, int R,
                                             const int32_t* seg_start, const int32_t* seg_pref,
@@ -554,8 +564,6 @@ __device__ __forceinline__ void fill_rowtab(int tile, int32_t* rowtab, int& cur_
   const int j0 = tile * kBN - before;
   while (cur_seg < nseg && seg_pref[cur_seg + 1] <= j0) ++cur_seg;
   const int j = j0 + lane;
-// `before` > 0: the tile starts that many positions ahead of tile * 64, and
-// positions below 0 (a mixed tile's current rows) get `past_end` too.
   int32_t row = past_end;
   if (j >= 0 && j < R) {
     int s = cur_seg;

@@ -292,12 +292,12 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
       return;
     }
   } else {
-    const int32_t ntiles = (w.R + kBN - 1) / kBN + ntc;
-    // A part needs kMinPartTiles key tiles to pay for its record and the
+    const int32_t ntiles = MIXED ? (w.R + L + kBN - 1) / kBN : (w.R + kBN - 1) / kBN + ntc;
+    // A part needs min_part key tiles to pay for its record and the
     // merge, so a short item runs as fewer parts (one, below two such runs);
     // every part of the item sees the same tile count and agrees.  Parts past
     // the count leave at once.
-    parts = ntiles / kMinPartTiles;
+    parts = ntiles / split.min_part;
     parts = parts < 1 ? 1 : (parts < un.parts ? parts : un.parts);
     if (un.part >= parts) return;
     t_begin = un.part * ntiles / parts;
@@ -538,7 +538,7 @@ hipError_t launch(const AttnArgs& a, const Scalars& s, hipStream_t st) {
   // With a workspace, some items are cut in two so the launch fills whole rounds of slots.
   int device = 0;
   const int32_t slots = a.workspace != nullptr && hipGetDevice(&device) == hipSuccess ? slots_of(device) : 0;
-  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0};
+  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0, 1};
   if (slots > 0 && a.workspace_bytes >= split_workspace_bytes(slots))
     split = round_split(static_cast<int32_t>(items), slots, (a.cur_len + kBN - 1) / kBN);
   AttnArgs b = a;

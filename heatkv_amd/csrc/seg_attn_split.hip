@@ -710,9 +710,9 @@ __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32
       te = p1 < tb ? tb : (p1 > ntiles ? ntiles : p1);
     }
   } else {
-    // as in the 16-bit kernel: a part needs kMinPartTiles tiles, parts past
+    // as in the 16-bit kernel: a part needs min_part tiles, parts past
     // the count leave at once
-    parts = ntiles / kMinPartTiles;
+    parts = ntiles / split.min_part;
     parts = parts < 1 ? 1 : (parts < un.parts ? parts : un.parts);
     if (un.part >= parts) return;
     tb = un.part * ntiles / parts;
@@ -870,7 +870,7 @@ hipError_t launch_half(const AttnArgs& a, const Scalars& s, hipStream_t st, int3
   if (items > 0x3fffffffLL) return hipErrorInvalidConfiguration;
   int device = 0;
   const int32_t slots = a.workspace != nullptr && hipGetDevice(&device) == hipSuccess ? split_slots(device) : 0;
-  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0};
+  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0, 1};
   if (slots > 0 && a.workspace_bytes >= split_workspace_bytes(slots))
     split = round_split(static_cast<int32_t>(items), slots, (a.cur_len + kBN - 1) / kBN);
   AttnArgs b = a;
