@@ -550,6 +550,10 @@ __device__ __forceinline__ int32_t xcd_item(int32_t j, int32_t groups, int32_t n
   return group * n_qt + qt;
 }
 
+// Current rows below which a kernel fills the last current tile with the first
+// prior rows (seg_attn_pipe_kernel, seg_attn_half_kernel: MIXED).
+constexpr int32_t kMixedBelow = 10 * kBN;
+
 // Row table of prior tile `tile` (wave 0, one entry per lane per 64 keys):
 // stream position -> slab row * ROW_BYTES, or `past_end` past R.  With
 // ROW_BYTES = 1 the entries are row indices.  `cur_seg` walks forward with

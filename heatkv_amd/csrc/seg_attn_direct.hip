@@ -105,8 +105,6 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 // 1000 tokens one tile in twenty no longer pays for the lanes' tests in the loop
 // (1023 tokens 41.0 / 41.8 planned, 4087 tokens 336 / 341 not planned): off from
 // kMixedBelow, and at multiples of 64, which have no such tile.
-constexpr int32_t kMixedBelow = 10 * kBN;  // current rows
-
 template <int QDT, int KDT, int VDT, bool MIXED>
 __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
     const int32_t* __restrict__ plan_p, const int32_t n_units, const AttnArgs a, const Scalars sc,

@@ -539,7 +539,13 @@ __device__ __forceinline__ uint32_t pack2_rest(float x, float y, uint32_t hi) {
 
 // `halves`: the plan's units are items of 256 queries, each run by two
 // workgroups (query halves) with the cut index 2 cut + half.
-template <int VDT>
+//
+// MIXED: tile nfull holds the current rows' last `rest` and the first prior
+// rows, as in the 16-bit kernel (seg_attn_pipe_kernel, where the lines of the
+// rule are drawn): its DMAs are issued for the lanes of current rows and again
+// for the lanes of prior rows.  With or without it, a last half without keys is
+// left out.
+template <int VDT, bool MIXED>
 __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32_t* __restrict__ plan_p,
                                                                     const int32_t n_units, const AttnArgs a,
                                                                     const Scalars sc, const int32_t n_qt,
@@ -619,6 +625,8 @@ __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32
   // current scale (b, h).
   const int64_t cur_row0 = static_cast<int64_t>(w.bh) * L;
   const int32_t ntc = (L + kBN - 1) / kBN;
+  const int32_t nfull = MIXED ? L / kBN : ntc;  // tiles from here on hold prior rows
+  const int32_t rest = MIXED ? L - nfull * kBN : 0;
   const u32x4_t dk_prior = make_desc(static_cast<const uint8_t*>(a.slab_k) + w.b * cap * kSRowBytes,
                                      static_cast<uint32_t>(cap * kSRowBytes));
   const u32x4_t dv_prior = make_desc(static_cast<const uint8_t*>(a.slab_v) + w.b * cap * Shape::kVRow,
@@ -638,35 +646,36 @@ __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32
   const int v_col = 2 * ((lane >> 5) * 32 + 16 * ((lp >> 3) & 1) + 8 * (lp & 1));
   const uint32_t ring_lds = lds_address(ring);
 
-  auto issue_k = [&](int j) {
+  // The half's current rows (`cur`) or prior rows; of the mixed tile the lanes
+  // of those (zeros past the stream's end).
+  auto issue_k_of = [&](int j, auto cur_tag) {
+    constexpr bool kCur = decltype(cur_tag)::value;
     const uint32_t dst = ring_lds + (j & 1) * kHKBytes + wave * 4 * 1024;
-    const int T = j >> 1;
+    const int T = j >> 1, key = (j & 1) * 32 + k_key;
+    if (MIXED && T == nfull && (key < rest) != kCur) return;
     int32_t off;
-    u32x4_t d;
-    if (T < ntc) {
+    if constexpr (kCur) {
       off = (j * 32 + k_key) * kSRowBytes + k_col;
-      d = dk_cur;
     } else {
-      const int32_t row = rowtab[(T - ntc) % 3][(j & 1) * 32 + k_key];
+      const int32_t row = rowtab[(T - nfull) % 3][key];
       off = row < 0 ? kPastEnd : row * kSRowBytes + k_col;
-      d = dk_prior;
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dma16(d, dst + i * 1024, off + i * 32);
+    for (int i = 0; i < 4; ++i) dma16(kCur ? dk_cur : dk_prior, dst + i * 1024, off + i * 32);
   };
-  auto issue_v = [&](int j) {
+  auto issue_v_of = [&](int j, auto cur_tag) {
+    constexpr bool kCur = decltype(cur_tag)::value;
     const uint32_t dst = ring_lds + 2 * kHKBytes + (j & 1) * Shape::kVBytes + wave * 2 * 1024;
-    const int T = j >> 1;
+    const int T = j >> 1, key = (j & 1) * 32 + v_key;
+    if (MIXED && T == nfull && (key < rest) != kCur) return;
     int32_t off;
-    u32x4_t d;
-    if (T < ntc) {
+    if constexpr (kCur) {
       off = (j * 32 + v_key) * Shape::kVRow + v_col;
-      d = dv_cur;
     } else {
-      const int32_t row = rowtab[(T - ntc) % 3][(j & 1) * 32 + v_key];
+      const int32_t row = rowtab[(T - nfull) % 3][key];
       off = row < 0 ? kPastEnd : row * Shape::kVRow + v_col;
-      d = dv_prior;
     }
+    const u32x4_t d = kCur ? dv_cur : dv_prior;
     dma16(d, dst, off);
     dma16(d, dst + 1024, off + 128);
     if constexpr (kSplitV) {
@@ -674,17 +683,28 @@ __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32
       dma16(d, dst + 32 * kD * 2 + 1024, off + kD * 2 + 128);
     }
   };
+  using Cur = std::integral_constant<bool, true>;
+  using Prior = std::integral_constant<bool, false>;
+  auto has_cur = [&](int j) { return MIXED ? (j >> 1) <= nfull : (j >> 1) < nfull; };
+  auto issue_k = [&](int j) {
+    if (has_cur(j)) issue_k_of(j, Cur{});
+    if ((j >> 1) >= nfull) issue_k_of(j, Prior{});
+  };
+  auto issue_v = [&](int j) {
+    if (has_cur(j)) issue_v_of(j, Cur{});
+    if ((j >> 1) >= nfull) issue_v_of(j, Prior{});
+  };
   // A unit whose first tile is a current-scale one (every whole item, and a
   // part that starts there) issues it, and Q, before the head's tables load:
   // tables, tile and Q arrive in one round trip.
   const int32_t first = cut ? (p0 < 0 ? 0 : p0) : 0;
   const bool early = planned && first < ntc;
-  auto issue_first = [&](int j) {
-    issue_k(j);
-    issue_v(j);
-    issue_k(j + 1);
+  auto issue_first = [&](int j, auto cur_tag) {
+    issue_k_of(j, cur_tag);
+    issue_v_of(j, cur_tag);
+    issue_k_of(j + 1, cur_tag);
   };
-  if (early) issue_first(2 * first);
+  if (early) issue_first(2 * first, Cur{});
 
   // Q in two bf16 pieces: B operands of S^T = K Q^T (query row, d = 16ks +
   // 8g .. +7); in flight while the tables load
@@ -701,7 +721,7 @@ __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32
     load_head_segments<kThreads>(a.seg_starts, a.seg_ends, a.seg_counts, cap, a.max_segments, w, seg_start,
                                  seg_pref);
   const int32_t R = w.R;
-  const int32_t ntiles = (R + kBN - 1) / kBN + ntc;
+  const int32_t ntiles = MIXED ? (L + R + kBN - 1) / kBN : (R + kBN - 1) / kBN + ntc;
   int32_t parts = un.parts;
   int32_t tb = 0, te = ntiles;
   if (planned) {
@@ -728,21 +748,26 @@ __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32
     return;
   }
 
-  auto valid_of = [&](int T) { return T < ntc ? min(kBN, L - T * kBN) : min(kBN, R - (T - ntc) * kBN); };
+  auto valid_of = [&](int T) {
+    if constexpr (MIXED) return min(kBN, L + R - T * kBN);
+    return T < ntc ? min(kBN, L - T * kBN) : min(kBN, R - (T - ntc) * kBN);
+  };
   int cur_seg = 0;
-  auto fill = [&](int T) {  // wave 0: row table of tile T (a prior-row tile)
-    if (T >= ntc && T < te)
-      fill_rowtab<1>(T - ntc, rowtab[(T - ntc) % 3], cur_seg, w.nseg, R, seg_start, seg_pref, -1);
+  auto fill = [&](int T) {  // wave 0: row table of tile T (one with prior rows)
+    if (T >= nfull && T < te)
+      fill_rowtab<1>(T - nfull, rowtab[(T - nfull) % 3], cur_seg, w.nseg, R, seg_start, seg_pref, -1, rest);
   };
 
   const int j0 = 2 * tb;
-  const int jend = 2 * te;
+  constexpr bool kOdd = MIXED || kSplitV;
+  const int jend = 2 * te - (kOdd && valid_of(te - 1) <= 32 ? 1 : 0);
   if (wave == 0) {
     fill(tb);
     fill(tb + 1);
   }
   __syncthreads();
-  if (!early) issue_first(j0);
+  if (!early && has_cur(j0)) issue_first(j0, Cur{});
+  if (tb >= nfull) issue_first(j0, Prior{});
 #pragma unroll
   for (int ks = 0; ks < 8; ++ks) {
     qh[ks] ^= sc.q_sign;
@@ -841,8 +866,13 @@ __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32
     step(More{}, sa, sb, j);
     step(More{}, sb, sa, j + 1);
   }
-  step(More{}, sa, sb, j);
-  step(Last{}, sb, sa, j + 1);
+  if (!kOdd || j + 1 < jend) {
+    step(More{}, sa, sb, j);
+    ++j;
+  } else {
+    sb = sa;  // an odd count: one Last step serves both (two spill registers)
+  }
+  step(Last{}, sb, sa, j);
 
   if (parts == 1) {
     if (a.out_dtype != kF32 && (reinterpret_cast<uintptr_t>(a.out) & 15) == 0) {
@@ -884,9 +914,13 @@ hipError_t launch_half(const AttnArgs& a, const Scalars& s, hipStream_t st, int3
   if (halves) grid = (grid + 7) / 8 * 16;
   if (grid <= 0) return hipSuccess;
   if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  seg_attn_half_kernel<VDT><<<dim3(static_cast<uint32_t>(grid)), kHThreads, 0, st>>>(
-      b.plan, b.plan != nullptr ? b.plan_units : 0, b, s, halves ? (a.cur_len + kSBM - 1) / kSBM : n_qt,
-      halves ? 1 : 0, split);
+  const int32_t units = b.plan != nullptr ? b.plan_units : 0;
+  const int32_t tiles = halves ? (a.cur_len + kSBM - 1) / kSBM : n_qt;
+  const dim3 blocks(static_cast<uint32_t>(grid));
+  if (a.cur_len % kBN != 0 && a.cur_len < kMixedBelow)
+    seg_attn_half_kernel<VDT, true><<<blocks, kHThreads, 0, st>>>(b.plan, units, b, s, tiles, halves ? 1 : 0, split);
+  else
+    seg_attn_half_kernel<VDT, false><<<blocks, kHThreads, 0, st>>>(b.plan, units, b, s, tiles, halves ? 1 : 0, split);
   return hipGetLastError();
 }
 

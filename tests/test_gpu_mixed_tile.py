@@ -1,4 +1,4 @@
-"""The 16-bit kernel's mixed tile: the last current rows and the first prior
+"""The mixed tile of the 16-bit and the split-row kernel: the last current rows and the first prior
 rows in one 64-key tile, at lengths and retained rows around the tile's edge,
 planned (whole, cut) and not, against the oracle."""
 
@@ -8,7 +8,8 @@ import numpy as np
 import pytest
 import torch
 
-from heatkv_amd import fused_real_pruning_flat_segmented_attention, segmented_attention_plan
+import heatkv_amd.real_pruning_fused_attention as op
+from heatkv_amd import attention_item_shape, fused_real_pruning_flat_segmented_attention, segmented_attention_plan
 from oracle import segmented_attention as oattn
 from support import assert_attention_close, to_np
 
@@ -16,9 +17,11 @@ pytestmark = pytest.mark.gpu
 SCALE = float(1.0 / np.sqrt(128.0))
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("qk,vt", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
+                                   (torch.float32, torch.bfloat16), (torch.float32, torch.float32)], ids=str)
 @pytest.mark.parametrize("L", [1, 8, 31, 33, 63, 65, 120, 129, 191, 639, 641])
-def test_mixed_tile_against_oracle(L, dtype, device):
+def test_mixed_tile_against_oracle(L, qk, vt, device, monkeypatch):
+    monkeypatch.setattr(op, "_SPLIT_VALUES_ROWS", 0)  # fp32 v: the split-row kernel at every size
     # per head: no prior rows, one, those that fill the tile less one / exactly
     # / plus one, a whole tile more, and many, in segments of uneven length
     rest = 64 - L % 64
@@ -32,8 +35,8 @@ def test_mixed_tile_against_oracle(L, dtype, device):
             at += cuts[i + 1] - cuts[i] + 2  # rows of no segment between
     ct = torch.full((H,), 3, dtype=torch.int32)
     g = torch.Generator().manual_seed(L)
-    q, ck, cv = (torch.randn((B, H, L, 128), generator=g).to(dtype) for _ in range(3))
-    sk, sv = (torch.randn((B, at, 128), generator=g).to(dtype) for _ in range(2))
+    q, ck, cv = (torch.randn((B, H, L, 128), generator=g).to(t) for t in (qk, qk, vt))
+    sk, sv = (torch.randn((B, at, 128), generator=g).to(t) for t in (qk, vt))
     live = torch.zeros(at, dtype=torch.bool)
     for s, e in zip(st.flatten().tolist(), en.flatten().tolist()):
         live[s:e] = True
@@ -42,11 +45,13 @@ def test_mixed_tile_against_oracle(L, dtype, device):
                                           st.numpy(), en.numpy(), ct.numpy(),
                                           *(to_np(t.float()) for t in (ck, cv)), SCALE)
     dev = [t.to(device) for t in (q, sk, sv, st, en, ct, ck, cv)]
+    queries, resident = attention_item_shape(qk, qk, vt, device=device)
     outs = {}
-    for name, slots in (("unplanned", None), ("planned", 512), ("cut", 4096)):
-        print(f"[attn] mixed tile L={L} {dtype} {name}", flush=True)
-        plan = None if slots is None else segmented_attention_plan(st, en, ct, batch_size=B, current_len=L,
-                                                                   capacity=at, device=device, slots=slots)
+    for name, slots in (("unplanned", None), ("planned", 1), ("cut", 16)):
+        print(f"[attn] mixed tile L={L} {qk} {vt} {name}", flush=True)
+        plan = None if slots is None else segmented_attention_plan(
+            st, en, ct, batch_size=B, current_len=L, capacity=at, device=device, queries_per_item=queries,
+            slots=slots * resident)
         out, lse = fused_real_pruning_flat_segmented_attention(
             q=dev[0], persisted_k=dev[1], persisted_v=dev[2], segment_starts=dev[3], segment_ends=dev[4],
             segment_counts=dev[5], current_k=dev[6], current_v=dev[7], softmax_scale=SCALE, return_lse=True,
