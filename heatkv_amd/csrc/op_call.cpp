@@ -149,19 +149,20 @@ bool plan_fits(PyObject* plan, int32_t queries, int64_t B, int64_t L, int dev, c
 
 // attention(q, persisted_k, persisted_v, segment_starts, segment_ends,
 // segment_counts, current_k, current_v, softmax_scale, softmax_mode,
-// return_lse, out_dtype, work_plan, k_split_rows, split_values_rows)
+// return_lse, out_dtype, work_plan, k_split_rows, split_values_rows,
+// split_values_slab_rows)
 PyObject* attention_call(PyObject* const* args, Py_ssize_t n) {
-  if (!g.ready || n != 15 || !no_modes() || knobs_set()) Py_RETURN_NONE;
+  if (!g.ready || n != 16 || !no_modes() || knobs_set()) Py_RETURN_NONE;
   const at::Tensor* t[8];
   for (int i = 0; i < 8; ++i)
     if ((t[i] = plain(args[i])) == nullptr) Py_RETURN_NONE;
   const at::Tensor &q = *t[0], &pk = *t[1], &pv = *t[2], &st = *t[3], &en = *t[4], &ct = *t[5], &ck = *t[6],
                    &cv = *t[7];
   double scale = 0;
-  int64_t split_rows_from = 0;
+  int64_t split_from = 0, split_slab = 0;
   bool with_lse = false, k_split = false;
   if (!number(args[8], &scale) || !flag(args[10], &with_lse) || !flag(args[13], &k_split) ||
-      !whole(args[14], &split_rows_from))
+      !whole(args[14], &split_from) || !whole(args[15], &split_slab))
     Py_RETURN_NONE;
   const char* mode = PyUnicode_CheckExact(args[9]) ? PyUnicode_AsUTF8(args[9]) : nullptr;
   if (mode == nullptr || (std::strcmp(mode, "exp") != 0 && std::strcmp(mode, "exp2") != 0)) {
@@ -197,7 +198,7 @@ PyObject* attention_call(PyObject* const* args, Py_ssize_t n) {
   // call itself unless the caller has them
   const bool rows32 = qc == HKV_DTYPE_F32 && vc != HKV_DTYPE_F32;
   if (k_split && !rows32) Py_RETURN_NONE;
-  const bool split_v = qc == HKV_DTYPE_F32 && vc == HKV_DTYPE_F32 && B * H * L >= split_rows_from;
+  const bool split_v = qc == HKV_DTYPE_F32 && vc == HKV_DTYPE_F32 && (B * H * L >= split_from || B * cap <= split_slab);
   const bool splits = (rows32 && !k_split) || split_v;
   if (splits && (!aligned(ck) || !aligned(pk) || (split_v && (!aligned(cv) || !aligned(pv))))) Py_RETURN_NONE;
   const int32_t queries = rows32 ? g.item_shape(qc, HKV_DTYPE_SPLIT_ROWS, vc, 1, 0, 0, 0, nullptr) : 128;

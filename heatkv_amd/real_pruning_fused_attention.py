@@ -145,23 +145,27 @@ def _split_rows_path(q_dtype, k_dtype, v_dtype, qk_mode: int, value_mode: int) -
             and qk_mode != 2 and value_mode != 2)
 
 
-# Current rows (batch x heads x length) from which all-fp32 calls split K and V
-# ahead of the attention.  The split-row kernel is the faster one at every size
-# (one image pair, 16 heads, device us with the split launch / staged kernel:
-# 36 tokens 16.3 / 16.8, 144: 27.3 / 29.2, 1024: 96 / 136, 2304: 320 / 537),
-# but below this a call is bound by its host work, which the split adds to
-# (a scratch tensor and a second launch, ~4 us).
+# All-fp32 calls split K and V ahead of the attention: faster than the staged
+# kernel at every size (one image pair, 16 heads, a tenth retained, whole calls,
+# us, split / staged: 4 tokens 10.4 / 16.0, 36: 13.3 / 16.4, 64: 15.3 / 16.2; one
+# image, 5 heads 144: 19.7 / 27.7, 400: 30.9 / 48.0; 2304 tokens, one pair: 305 /
+# 538).  The copies hold a row for every slab row, so where the slab is large
+# (64 MB of copies) and the call small (fewer current rows, batch x heads x
+# length, than this), the staged kernel's call without them stays.
 _SPLIT_VALUES_ROWS = 4096
+_SPLIT_VALUES_SLAB_ROWS = 65536
 
 
-def _split_values_path(q, k, v, qk_mode: int, value_mode: int) -> bool:
-    """fp32 q, k and v at the default (or tf32) dot modes, with enough rows, run
-    the split-row kernel's 128-query form on split copies of K and V; otherwise
-    (and with HKV_ATTN_SPLIT_ROWS=0) the register-staged kernel, which splits
-    every tile for every query tile itself."""
+def _split_values_path(q, k, v, slab_k, qk_mode: int, value_mode: int) -> bool:
+    """fp32 q, k and v at the default (or tf32) dot modes run the split-row
+    kernel's 128-query form on split copies of K and V; otherwise (and for small
+    calls on very large slabs, and with HKV_ATTN_SPLIT_ROWS=0) the
+    register-staged kernel, which splits every tile for every query tile itself."""
     return (q.dtype == torch.float32 and k.dtype == torch.float32 and v.dtype == torch.float32
             and qk_mode != 2 and value_mode != 2
-            and q.shape[0] * q.shape[1] * q.shape[2] >= _SPLIT_VALUES_ROWS and _split_rows_enabled())
+            and (q.shape[0] * q.shape[1] * q.shape[2] >= _SPLIT_VALUES_ROWS
+                 or slab_k.shape[0] * slab_k.shape[1] <= _SPLIT_VALUES_SLAB_ROWS)
+            and _split_rows_enabled())
 
 
 def split_rows_k_format(q_dtype, k_dtype, v_dtype) -> bool:
@@ -460,7 +464,7 @@ def fused_real_pruning_flat_segmented_attention(
     if native is not None and append_offsets is None and append_also is None and _bind is None:
         out = native.attention(q, persisted_k, persisted_v, segment_starts, segment_ends, segment_counts, current_k,
                                current_v, softmax_scale, softmax_mode, return_lse, out_dtype, work_plan, k_split_rows,
-                               _SPLIT_VALUES_ROWS)
+                               _SPLIT_VALUES_ROWS, _SPLIT_VALUES_SLAB_ROWS)
         if out is not None:
             return out
     if q.ndim != 4 or current_k.ndim != 4 or current_v.ndim != 4:
@@ -555,7 +559,7 @@ def fused_real_pruning_flat_segmented_attention(
     if k_split_rows:
         _check_split_rows_k(q.dtype, current_k.dtype, current_v.dtype, qk_mode, value_mode)
     split = k_split_rows or _split_rows_path(q.dtype, current_k.dtype, current_v.dtype, qk_mode, value_mode)
-    split_v = not split and _split_values_path(q, current_k, current_v, qk_mode, value_mode)
+    split_v = not split and _split_values_path(q, current_k, current_v, persisted_k, qk_mode, value_mode)
     if work_plan is not None:
         if (work_plan.dtype != torch.int32 or work_plan.ndim != 2 or work_plan.shape[1] != PLAN_INTS
                 or not work_plan.is_contiguous()):
