@@ -513,6 +513,354 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
                              ring + wave * 32 * kOutPitch);
 }
 
+// ---------------------------------------------------------------- small launches
+//
+// The same stream (with its mixed tile), products and softmax for launches of
+// up to one workgroup per CU at up to kSmallMaxLen queries: 64-query items, 4
+// waves x 16 queries on the 16x16x32 MFMAs.  Such a launch is bound by its
+// chain of round trips and by the serial chain of a tile, not by throughput.
+//  * A ring of four whole tiles: those of current rows go out before the
+//    head's tables arrive, three in flight; a wait counts the DMAs of the tiles
+//    behind its own (8 or more each per wave: in the mixed tile every one of
+//    the 8 is issued for one kind of lane at least; what was issued before q
+//    has landed with it).
+//  * S(t + 1) = K(t + 1) Q^T runs while the VALU turns S(t) into P(t), as in
+//    seg_attn_pipe_kernel.  Half the queries per wave halve a tile's MFMAs and
+//    exponentials, but not its LDS reads (1024 of ~2000 cycles with four
+//    waves), so longer items gain nothing.
+//  * K rows and V rows lie in LDS as in seg_attn_pipe_kernel.  K operand
+//    (16 keys x 32 d) of key block kb, step ks: lane l holds K[16 kb + l % 16]
+//    [32 ks + 8 (l / 16) .. + 7].  The P operand of a 32-key step takes its k
+//    slots 8 g .. 8 g + 7 (g = l / 16) as keys 4 g .. + 3 and 16 + 4 g .. + 3,
+//    which is how S^T leaves the MFMA, and the V operand is read in that order.
+//  * A plan's 128-query units are run by two workgroups each, 8 ids apart (on
+//    one XCD).
+// us, seg_attn_pipe_kernel / here, B=2, 16 heads, a tenth retained: not planned
+// 4 tokens 7.8 / 6.8, 16: 7.9 / 6.9, 36: 8.5 / 7.4, 64: 9.4 / 8.1, 144: 11.2 / 9.9;
+// planned 6.5 / 6.1, 6.9 / 6.3, 7.1 / 6.6, 8.2 / 7.5, 10.2 / 9.7.  256 tokens,
+// uneven heads: 15.4 / 16.4 not planned; 400: 19.9 / 30 planned, which cuts its
+// longest items.
+template <int MT>
+__device__ __forceinline__ f32x4_t mfma16(u32x4_t a, u32x4_t b, f32x4_t c) {
+  if constexpr (MT == kF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c,
+                                                  0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
+                                                   c, 0, 0, 0);
+}
+
+// Maximum / sum over the four lanes l, l ^ 16, l ^ 32, l ^ 48 of a query.
+__device__ __forceinline__ float quad_max(float v) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  return pair_max(fmaxf(__builtin_bit_cast(float, static_cast<uint32_t>(r[0])),
+                        __builtin_bit_cast(float, static_cast<uint32_t>(r[1]))));
+}
+__device__ __forceinline__ float quad_sum(float v) {
+  const uint32_t b = __builtin_bit_cast(uint32_t, v);
+  const auto r = __builtin_amdgcn_permlane16_swap(b, b, false, false);
+  return pair_sum(__builtin_bit_cast(float, static_cast<uint32_t>(r[0])) +
+                  __builtin_bit_cast(float, static_cast<uint32_t>(r[1])));
+}
+
+constexpr int kSmallBM = 64;
+constexpr int32_t kSmallMaxLen = 3 * kBN;
+constexpr int32_t kSmallRowsPerHead = 256;
+
+inline int64_t items_of(const AttnArgs& a, int32_t queries) {
+  return static_cast<int64_t>(a.batch) * a.heads * ((a.cur_len + queries - 1) / queries);
+}
+
+// Whether a launch runs seg_attn_small_kernel: few queries, a CU per 64-query
+// item, and items that seg_attn_pipe_kernel would not cut either -- a plan
+// without cut items (one unit per item), or no plan and a slab that holds few
+// rows per head (the rows that the tables retain are not known here; with
+// many, the parts of the round split are shorter than a whole item).
+inline bool small_launch(const AttnArgs& a, int64_t items, int32_t cus) {
+  if (a.cur_len > kSmallMaxLen || items_of(a, kSmallBM) > cus) return false;
+  return a.plan != nullptr ? a.plan_units == items
+                           : a.slab_capacity <= static_cast<int64_t>(kSmallRowsPerHead) * a.heads;
+}
+
+template <int DT, int VDT>
+__global__ __launch_bounds__(256, 1) void seg_attn_small_kernel(const int32_t* __restrict__ plan_p,
+                                                                const int32_t n_units, const AttnArgs a,
+                                                                const Scalars sc) {
+  constexpr int kThreads = 256;
+  constexpr int NS = 4;
+  __shared__ __attribute__((aligned(1024))) uint8_t ring[NS * kStageBytes];
+  __shared__ __attribute__((aligned(16))) int32_t rowtab[NS][kBN];
+  __shared__ int32_t seg_start[kMaxSegments];
+  __shared__ int32_t seg_pref[kMaxSegments + 1];
+  static_assert(NS * kStageBytes >= 2 * kMaxHeads * 4, "head tables alias the ring");
+
+  if (a.append_offsets != nullptr && static_cast<int32_t>(blockIdx.x) >= a.append_first) {
+    append_block<256>(a, blockIdx.x - static_cast<uint32_t>(a.append_first), kD * 2, kD * 2);
+    return;
+  }
+  const int64_t cap = a.slab_capacity;
+  const int H = a.heads;
+  const int L = a.cur_len;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int g = lane >> 4;
+  const int32_t n_qt = (L + kSmallBM - 1) / kSmallBM;
+
+  WorkItem w;
+  const bool planned = plan_p != nullptr;
+  if (planned) {
+    const int32_t id = static_cast<int32_t>(blockIdx.x);
+    const int32_t uid = ((id >> 4) << 3) + (id & 7);
+    if (uid >= n_units) return;
+    const int32_t* pu = plan_p + static_cast<int64_t>(uid) * kPlanInts;
+    const int32_t ph = pu[0], pj = pu[1];
+    const int32_t n_qt2 = (L + 127) / 128;
+    if (ph < 0 || ph >= H || pj < 0 || pj >= a.batch * n_qt2) return;  // not a unit of this launch
+    w.h = ph;
+    w.b = pj / n_qt2;
+    w.qt = 2 * (pj - w.b * n_qt2) + ((id >> 3) & 1);
+    if (w.qt >= n_qt) return;
+    w.bh = w.b * H + w.h;
+  } else {
+    int32_t* head_rows = reinterpret_cast<int32_t*>(ring);
+    const int32_t item = xcd_item(static_cast<int32_t>(blockIdx.x), a.batch * H, n_qt);
+    w = plan_work<kThreads>(a.seg_starts, a.seg_ends, a.seg_counts, cap, H, a.max_segments, a.batch, n_qt, head_rows,
+                            head_rows + kMaxHeads, seg_start, seg_pref, item, head_rows + 2 * kMaxHeads,
+                            NS * kStageBytes / 4 - 2 * kMaxHeads);
+  }
+
+  // waves 0 and 1 load K, waves 2 and 3 V, 8 DMAs a tile each, in
+  // seg_attn_pipe_kernel's pattern
+  const bool k_wave = wave < 2;
+  const int64_t cur_row0 = static_cast<int64_t>(w.bh) * L;
+  const u32x4_t d_prior = make_desc(
+      static_cast<const uint8_t*>(k_wave ? a.slab_k : a.slab_v) + static_cast<int64_t>(w.b) * cap * kD * 2,
+      static_cast<uint32_t>(cap * kD * 2));
+  const u32x4_t d_cur = make_desc(static_cast<const uint8_t*>(k_wave ? a.cur_k : a.cur_v) + cur_row0 * kD * 2,
+                                  static_cast<uint32_t>(L * kD * 2));
+  constexpr int32_t kPastEnd = static_cast<int32_t>(0x80000000u);
+  int key0, col0;
+  if (k_wave) {
+    key0 = wave * 32 + (lane & 31);
+    col0 = (lane >> 5) * 16;
+  } else {
+    const int lp = lane & 31;
+    key0 = 32 * (wave - 2) + 4 * (lp >> 4) + ((lp & 7) >> 1);
+    col0 = 2 * ((lane >> 5) * 32 + 16 * ((lp >> 3) & 1) + 8 * (lp & 1));
+  }
+  const uint32_t ring_lds = lds_address(ring) + wave * 8 * 1024;
+  const int32_t nfull = L / kBN;           // tiles of current rows only
+  const int32_t rest = L - nfull * kBN;    // current rows of tile nfull
+
+  // rows of one kind of a tile, for the lanes with key in [from, lim): byte
+  // offsets of keys key0, + 8, + 16, + 24 (K waves: key0 only)
+  auto issue_rows = [&](int t, const u32x4_t d, const int32_t (&off)[4], int from, int lim) {
+    const uint32_t dst = ring_lds + (t % NS) * kStageBytes;
+    if (k_wave) {
+      if (key0 >= from && key0 < lim) {
+        dma16_at<0>(d, dst, off[0]);
+        dma16_at<32>(d, dst + 1024, off[0]);
+        dma16_at<64>(d, dst + 2048, off[0]);
+        dma16_at<96>(d, dst + 3072, off[0]);
+        dma16_at<128>(d, dst + 4096, off[0]);
+        dma16_at<160>(d, dst + 5120, off[0]);
+        dma16_at<192>(d, dst + 6144, off[0]);
+        dma16_at<224>(d, dst + 7168, off[0]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        if (key0 + 8 * i >= from && key0 + 8 * i < lim) {
+          dma16_at<0>(d, dst + 2048 * i, off[i]);
+          dma16_at<128>(d, dst + 2048 * i + 1024, off[i]);
+        }
+    }
+  };
+  auto issue_cur = [&](int t) {
+    int32_t off[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) off[i] = (t * kBN + key0 + 8 * i) * (kD * 2) + col0;
+    issue_rows(t, d_cur, off, 0, t < nfull ? kBN : rest);
+  };
+  auto issue_prior = [&](int t) {
+    int32_t off[4];
+    const int32_t* rt = rowtab[t % NS];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) off[i] = rt[key0 + (k_wave ? 0 : 8 * i)] + col0;
+    issue_rows(t, d_prior, off, t > nfull ? 0 : rest, kBN);
+  };
+  const int32_t cur_tiles = nfull + (rest > 0 ? 1 : 0);
+  if (planned)
+    for (int t = 0; t < NS - 1 && t < cur_tiles; ++t) issue_cur(t);
+
+  const int32_t qrow = w.qt * kSmallBM + wave * 16 + (lane & 15);
+  u32x4_t qf[4];
+  {
+    const __amdgpu_buffer_rsrc_t rq = make_rsrc(
+        static_cast<const uint8_t*>(a.q) + cur_row0 * kD * 2, static_cast<uint32_t>(L * kD * 2));
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) qf[ks] = load8<DT, DT>(rq, qrow < L ? (qrow * kD + ks * 32 + g * 8) * 2 : -1);
+  }
+  if (planned)
+    load_head_segments<kThreads>(a.seg_starts, a.seg_ends, a.seg_counts, cap, a.max_segments, w, seg_start,
+                                 seg_pref);
+  const int32_t R = w.R;
+  const int32_t ntiles = (L + R + kBN - 1) / kBN;
+  int cur_seg = 0;
+  auto fill = [&](int t) {  // wave 0: row table of tile t, if it holds prior rows
+    if (t >= nfull && t < ntiles)
+      fill_rowtab<kD * 2>(t - nfull, rowtab[t % NS], cur_seg, w.nseg, R, seg_start, seg_pref, kPastEnd, rest);
+  };
+  if (wave == 0)
+    for (int t = 0; t < NS; ++t) fill(t);
+  __syncthreads();
+  // q lands here, and with it everything issued so far: the rest of the
+  // prologue's tiles go out behind it
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    qf[ks] ^= sc.q_sign;
+    asm volatile("" : "+v"(qf[ks]));
+  }
+  for (int t = 0; t < NS - 1 && t < ntiles; ++t) {
+    if (!planned && t < cur_tiles) issue_cur(t);
+    if (t >= nfull) issue_prior(t);
+  }
+
+  f32x4_t oacc[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) oacc[i] = f32x4_t{};
+  float m_run = -1e30f;
+  float l_run = 0.f;
+  const uint8_t* const k_lane = ring + (lane >> 5) * 1024 + ((lane & 15) + 32 * (g & 1)) * 16;
+  const uint8_t* const v_lane = ring + kTileBytes + (g >> 1) * 2048 + (g & 1) * 256 + (lane & 15) * 8;
+
+  auto qk = [&](f32x4_t (&s)[4], int t) {
+    const uint8_t* const kst = k_lane + (t % NS) * kStageBytes;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) s[kb] = f32x4_t{};
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        const u32x4_t kf =
+            *reinterpret_cast<const u32x4_t*>(kst + (kb >> 1) * 8192 + ks * 2048 + (kb & 1) * 256);
+        s[kb] = mfma16<DT>(kf, qf[ks], s[kb]);
+      }
+  };
+  // the row max of S(t) moves the running one
+  auto take_max = [&](f32x4_t (&s)[4], int t) {
+    const int valid = L + R - t * kBN;
+    if (valid < kBN) {
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (16 * kb + j >= valid - 4 * g) s[kb][j] = -__builtin_inff();
+    }
+    float mx = s[0][0];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) mx = fmaxf(mx, s[kb][j]);
+    mx = quad_max(mx);
+    if (__any(mx - m_run > sc.thresh)) {
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * sc.c);
+      l_run *= alpha;
+#pragma unroll
+      for (int db = 0; db < 8; ++db) oacc[db] *= alpha;
+      m_run = m_new;
+    }
+  };
+  auto exps = [&](f32x4_t (&s)[4]) {
+    const float mc = m_run * sc.c;
+    float psum[4];
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) s[kb][j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[kb][j], sc.c, -mc));
+      psum[kb] = (s[kb][0] + s[kb][1]) + (s[kb][2] + s[kb][3]);
+    }
+    l_run += (psum[0] + psum[1]) + (psum[2] + psum[3]);
+  };
+  auto pv = [&](const f32x4_t (&s)[4], int t) {
+    const uint8_t* const vst = v_lane + (t % NS) * kStageBytes;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      u32x4_t pf;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        pf[2 * i] = pack2<VDT>(s[2 * u + i][0], s[2 * u + i][1]);
+        pf[2 * i + 1] = pack2<VDT>(s[2 * u + i][2], s[2 * u + i][3]);
+      }
+#pragma unroll
+      for (int db = 0; db < 8; ++db) {
+        const uint8_t* const blk = vst + u * 8192 + (db >> 2) * 1024 + ((db >> 1) & 1) * 512 + (db & 1) * 128;
+        const u32x2_t lo = ds_read_tr(blk);
+        const u32x2_t hi = ds_read_tr(blk + 4096);
+        const u32x4_t vf = {lo[0], lo[1], hi[0], hi[1]};
+        oacc[db] = mfma16<VDT>(vf, pf, oacc[db]);
+      }
+    }
+  };
+  // the DMAs of at most `behind` tiles outstanding
+  auto wait_tiles = [&](int behind) {
+    if (behind >= 2) wait_vmcnt<16>();
+    else if (behind == 1) wait_vmcnt<8>();
+    else wait_vmcnt<0>();
+  };
+  // tile 0: of the NS - 1 issued, NS - 2 may be in flight
+  wait_tiles(min(NS - 2, ntiles - 1));
+  __syncthreads();
+  f32x4_t sa[4], sb[4];
+  qk(sa, 0);
+  take_max(sa, 0);
+  auto step = [&](f32x4_t (&scur)[4], f32x4_t (&snext)[4], int t) {
+    wait_tiles(min(NS - 3, ntiles - 2 - t));  // tile t + 1 landed
+    __syncthreads();  // and every wave is past tile t - 1, whose stage is next
+    const int next = t + NS - 1;
+    if (next < ntiles) {
+      if (next < cur_tiles) issue_cur(next);
+      if (next >= nfull) issue_prior(next);
+    }
+    if (wave == 0) fill(t + NS);
+    qk(snext, t + 1);
+    exps(scur);
+    pv(scur, t);
+    take_max(snext, t + 1);
+  };
+  int t = 0;
+  for (; t + 2 < ntiles; t += 2) {
+    step(sa, sb, t);
+    step(sb, sa, t + 1);
+  }
+  if (t + 1 < ntiles) {
+    step(sa, sb, t);
+    ++t;
+#pragma unroll
+    for (int kb = 0; kb < 4; ++kb) sa[kb] = sb[kb];
+  }
+  exps(sa);
+  pv(sa, t);
+
+  const float l_tot = quad_sum(l_run);
+  const float inv = 1.f / l_tot;
+  if (qrow >= L) return;
+  const int64_t out_row = (static_cast<int64_t>(w.b) * L + qrow) * (static_cast<int64_t>(H) * kD) + w.h * kD;
+#pragma unroll
+  for (int db = 0; db < 8; ++db) {
+    const f32x4_t v = oacc[db] * inv;
+    const int64_t at = out_row + db * 16 + 4 * g;
+    if (a.out_dtype == kF32) store4<kF32>(a.out, at, v);
+    else if (a.out_dtype == kF16) store4<kF16>(a.out, at, v);
+    else store4<kBF16>(a.out, at, v);
+  }
+  if (a.lse != nullptr && g == 0)
+    a.lse[static_cast<int64_t>(w.bh) * L + qrow] = (m_run * sc.c + __log2f(l_tot)) * 0.6931471805599453f;
+}
+
 // Resident workgroups of the kernel (2 per CU) on `device`, cached.
 int32_t slots_of(int device) {
   static int32_t cache[64] = {};
@@ -530,12 +878,13 @@ template <int DT, int VDT>
 hipError_t launch(const AttnArgs& a, const Scalars& s, hipStream_t st) {
   constexpr int kBM = 128;
   const int32_t n_qt = (a.cur_len + kBM - 1) / kBM;
-  const int64_t items = static_cast<int64_t>(a.batch) * a.heads * n_qt;
+  const int64_t items = items_of(a, kBM);
   if (items <= 0) return hipSuccess;
   if (items > 0x3fffffffLL) return hipErrorInvalidConfiguration;
   // With a workspace, some items are cut in two so the launch fills whole rounds of slots.
   int device = 0;
-  const int32_t slots = a.workspace != nullptr && hipGetDevice(&device) == hipSuccess ? slots_of(device) : 0;
+  const int32_t cus = hipGetDevice(&device) == hipSuccess ? slots_of(device) / 2 : 0;
+  const int32_t slots = a.workspace != nullptr ? slots_of(device) : 0;
   RoundSplit split{static_cast<int32_t>(items), 0, 0, 0, 1};
   if (slots > 0 && a.workspace_bytes >= split_workspace_bytes(slots))
     split = round_split(static_cast<int32_t>(items), slots, (a.cur_len + kBN - 1) / kBN);
@@ -550,6 +899,14 @@ hipError_t launch(const AttnArgs& a, const Scalars& s, hipStream_t st) {
   const int64_t blocks = a.plan != nullptr ? (a.plan_units > 0 ? a.plan_units : 0) : split_units(split);
   if (blocks + copies <= 0) return hipSuccess;
   if (blocks + copies > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  if (small_launch(a, items, cus)) {
+    const int64_t small = a.plan != nullptr ? (blocks + 7) / 8 * 16 : items_of(a, kSmallBM);
+    if (small + copies > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+    b.append_first = static_cast<int32_t>(small);
+    seg_attn_small_kernel<DT, VDT><<<dim3(static_cast<uint32_t>(small + copies)), 256, 0, st>>>(
+        b.plan, b.plan != nullptr ? b.plan_units : 0, b, s);
+    return hipGetLastError();
+  }
   b.append_first = static_cast<int32_t>(blocks);
   const dim3 grid(static_cast<uint32_t>(blocks + copies));
   const int32_t units = b.plan != nullptr ? static_cast<int32_t>(blocks) : 0;

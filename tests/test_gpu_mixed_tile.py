@@ -1,4 +1,5 @@
-"""The mixed tile of the 16-bit and the split-row kernel: the last current rows and the first prior
+"""The mixed tile of the 16-bit kernels (128-query items, and 64-query items for
+few queries without cut items) and the split-row kernel: the last current rows and the first prior
 rows in one 64-key tile, at lengths and retained rows around the tile's edge,
 planned (whole, cut) and not, against the oracle."""
 
@@ -19,7 +20,7 @@ SCALE = float(1.0 / np.sqrt(128.0))
 
 @pytest.mark.parametrize("qk,vt", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16),
                                    (torch.float32, torch.bfloat16), (torch.float32, torch.float32)], ids=str)
-@pytest.mark.parametrize("L", [1, 8, 31, 33, 63, 65, 120, 129, 191, 639, 641])
+@pytest.mark.parametrize("L", [1, 8, 16, 31, 33, 63, 64, 65, 120, 128, 129, 191, 192, 193, 639, 641])
 def test_mixed_tile_against_oracle(L, qk, vt, device, monkeypatch):
     monkeypatch.setattr(op, "_SPLIT_VALUES_ROWS", 0)  # fp32 v: the split-row kernel at every size
     # per head: no prior rows, one, those that fill the tile less one / exactly
@@ -47,7 +48,7 @@ def test_mixed_tile_against_oracle(L, qk, vt, device, monkeypatch):
     dev = [t.to(device) for t in (q, sk, sv, st, en, ct, ck, cv)]
     queries, resident = attention_item_shape(qk, qk, vt, device=device)
     outs = {}
-    for name, slots in (("unplanned", None), ("planned", 1), ("cut", 16)):
+    for name, slots in (("unplanned", None), ("planned", 1), ("cut", 16), ("whole", 0)):
         print(f"[attn] mixed tile L={L} {qk} {vt} {name}", flush=True)
         plan = None if slots is None else segmented_attention_plan(
             st, en, ct, batch_size=B, current_len=L, capacity=at, device=device, queries_per_item=queries,
