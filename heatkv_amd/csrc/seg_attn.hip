@@ -53,15 +53,11 @@ hipError_t launch_segmented_attention(const AttnArgs& a, hipStream_t stream) {
   s.c = fmaxf(scale_abs * attn::kLog2e, attn::kMinC);
   s.thresh = attn::kRescaleLog2 / s.c;
   s.q_sign = a.softmax_scale < 0.f ? 0x80008000u : 0u;
-  hipError_t e;
-  if (a.k_dtype == kSplitRows) {
-    e = launch_attention_split(a, s, stream);
-  } else {
-    if (a.q_dtype != a.k_dtype) return hipErrorInvalidValue;
-    // the 16-bit kernel runs the append in its own launch
-    if (!force_staged() && attention_direct_supported(a)) return launch_attention_direct(a, s, stream);
-    e = launch_attention_staged(a, s, stream);
-  }
+  // the split-row and 16-bit kernels see to the append themselves
+  if (a.k_dtype == kSplitRows) return launch_attention_split(a, s, stream);
+  if (a.q_dtype != a.k_dtype) return hipErrorInvalidValue;
+  if (!force_staged() && attention_direct_supported(a)) return launch_attention_direct(a, s, stream);
+  const hipError_t e = launch_attention_staged(a, s, stream);
   if (e != hipSuccess || a.append_offsets == nullptr) return e;
   return launch_append(a, stream);
 }

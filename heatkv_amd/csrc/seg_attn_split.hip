@@ -564,6 +564,11 @@ __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32
   static_assert(Shape::kRing >= kHW * 32 * kOutPitch, "output staging fits the ring");
   static_assert(kPartialFloats == 66 * kThreads, "partial record layout");
 
+  if (a.append_offsets != nullptr && static_cast<int32_t>(blockIdx.x) >= a.append_first) {
+    // a copy block of the fused append, after the attention workgroups
+    append_block<kThreads>(a, blockIdx.x - static_cast<uint32_t>(a.append_first), kSRowBytes, Shape::kVRow);
+    return;
+  }
   // This workgroup's plan unit.  Two workgroups of a 256-query unit sit 8 ids
   // apart: on one XCD, as the plan dealt the unit.
   int32_t uid = static_cast<int32_t>(blockIdx.x);
@@ -916,7 +921,10 @@ hipError_t launch_half(const AttnArgs& a, const Scalars& s, hipStream_t st, int3
   if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
   const int32_t units = b.plan != nullptr ? b.plan_units : 0;
   const int32_t tiles = halves ? (a.cur_len + kSBM - 1) / kSBM : n_qt;
-  const dim3 blocks(static_cast<uint32_t>(grid));
+  const int64_t copies = a.append_offsets != nullptr ? append_blocks(a.batch, a.heads, a.cur_len) : 0;
+  if (grid + copies > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+  b.append_first = static_cast<int32_t>(grid);
+  const dim3 blocks(static_cast<uint32_t>(grid + copies));
   if (a.cur_len % kBN != 0 && a.cur_len < kMixedBelow)
     seg_attn_half_kernel<VDT, true><<<blocks, kHThreads, 0, st>>>(b.plan, units, b, s, tiles, halves ? 1 : 0, split);
   else
@@ -975,6 +983,8 @@ bool attention_split_supported(const AttnArgs& a) {
          a.qk_dot_mode != kDotFp32 && a.value_dot_mode != kDotFp32;
 }
 
+// The append rides in the 128-query form's launch (a layer's early and middle
+// scales, where a launch of its own costs 2-3 us) and follows the 256-query one.
 hipError_t launch_attention_split(const AttnArgs& a, const attn::Scalars& s, hipStream_t stream) {
   if (a.v_dtype == kSplitRows) {  // only from hkv_segmented_attention_split: plans of 128-query items
     if (a.q_dtype != kF32 || a.k_dtype != kSplitRows) return hipErrorInvalidValue;
@@ -983,7 +993,8 @@ hipError_t launch_attention_split(const AttnArgs& a, const attn::Scalars& s, hip
   if (!attention_split_supported(a)) return hipErrorInvalidValue;
   if (split_in_halves(a))
     return a.v_dtype == kBF16 ? launch_half<kBF16>(a, s, stream, kSBM) : launch_half<kF16>(a, s, stream, kSBM);
-  return a.v_dtype == kBF16 ? launch<kBF16>(a, s, stream) : launch<kF16>(a, s, stream);
+  const hipError_t e = a.v_dtype == kBF16 ? launch<kBF16>(a, s, stream) : launch<kF16>(a, s, stream);
+  return e != hipSuccess || a.append_offsets == nullptr ? e : launch_append(a, stream);
 }
 
 hipError_t launch_split_operands(SplitOperands o, bool with_v, hipStream_t stream) {
