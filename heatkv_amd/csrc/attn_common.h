@@ -457,6 +457,12 @@ __device__ __forceinline__ WorkItem plan_work(const int32_t* __restrict__ seg_st
 // once would leave half of the XCDs idle.  (Measured on the 2B scales:
 // adjacent parts run scale 9 in 36 us against 40 us grouped; grouped parts
 // run scale 8 in 21 us against 30 us adjacent.)
+// Where every item is cut and the parts fill one round of more units than CUs,
+// the first half of the workgroups runs in reverse order (mirror): workgroups i
+// and i + G / 2 share a CU, and the heaviest of the second half then joins the
+// lightest of the first (1600 tokens, B=1, 16 heads: 45.1 -> 42.0 us, uneven heads
+// 47.0 -> 43.7; fp32 q/k 67.6 -> 63.2, 70.3 -> 64.0; 1024 tokens, B=2: 40.7 / 40.7).
+//
 // Key tiles a part of a cut item must have at least (min_part): 5, or 4 where
 // every part has a CU to itself (a quarter of the slots).  16 heads, not
 // planned, us at 8 / 5 / 4 tiles: 576 tokens, B=2 25.8 / 22.1 / 23.9 (fp32 q/k
@@ -473,18 +479,20 @@ struct RoundSplit {
   int32_t grouped;      // first parts, then second parts (else each item's two parts adjacent)
   int32_t whole_first;  // whole items before the cut items' parts
   int32_t min_part;     // key tiles of a part at least
+  int32_t mirror;       // workgroups [0, mirror) in reverse order (0: none)
 };
 
 // `min_tiles`: key tiles every item has at least (its current-scale tiles).
 __host__ __device__ __forceinline__ RoundSplit round_split(int32_t items, int32_t slots, int32_t min_tiles) {
   const int32_t min_part = 4LL * items <= slots ? kMinPartTilesAlone : kMinPartTiles;
-  RoundSplit t{items, 0, min_tiles < 2 * min_part ? 1 : 0, 0, min_part};
+  RoundSplit t{items, 0, min_tiles < 2 * min_part ? 1 : 0, 0, min_part, 0};
   if (slots <= 0 || items >= 2 * slots) return t;
   if (items > slots) {
     t.two = 2 * slots - items;
     t.whole_first = 1;
   } else {
     t.two = items < slots - items ? items : slots - items;
+    if (t.two == items && t.grouped == 0 && 4LL * items > slots) t.mirror = slots / 2;
   }
   return t;
 }
@@ -506,6 +514,7 @@ struct Unit {
 };
 
 __host__ __device__ __forceinline__ Unit split_unit(const RoundSplit& t, int32_t j) {
+  if (j < t.mirror) j = t.mirror - 1 - j;
   Unit u{j, 0, 1, 0, 0, 0};
   if (t.two == 0) return u;
   const int32_t lead = t.whole_first ? t.items - t.two : 0;  // whole items before the parts

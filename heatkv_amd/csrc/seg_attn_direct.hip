@@ -107,7 +107,7 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 // kMixedBelow, and at multiples of 64, which have no such tile.
 template <int QDT, int KDT, int VDT, bool MIXED>
 __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
-    const int32_t* __restrict__ plan_p, const int32_t n_units, const AttnArgs a, const Scalars sc,
+    const int32_t* __restrict__ plan_p, const int32_t units_arg, const AttnArgs a, const Scalars sc,
     const int32_t n_qt, const RoundSplit split) {
   static_assert(KDT != kF32 && VDT != kF32 && QDT == KDT, "16-bit inputs only");
   constexpr int NW = 4;
@@ -132,9 +132,14 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
   // out with the other kernel arguments' loads instead of after them (about
   // 0.5 us less per launch on the small scales).
   int32_t pu[kPlanInts] = {};
-  const bool planned = plan_p != nullptr && static_cast<int32_t>(blockIdx.x) < n_units;
+  // units_arg < 0: bits 16 .. 30 hold the workgroups that take the plan's units
+  // in reverse order (launch), the low 16 the unit count.
+  const int32_t mirror = units_arg < 0 ? (units_arg >> 16) & 0x7fff : 0;
+  const int32_t n_units = units_arg < 0 ? units_arg & 0xffff : units_arg;
+  const int32_t uid = static_cast<int32_t>(blockIdx.x);
+  const bool planned = plan_p != nullptr && uid < n_units;
   if (planned) {
-    const int32_t* src = plan_p + static_cast<int64_t>(blockIdx.x) * kPlanInts;
+    const int32_t* src = plan_p + static_cast<int64_t>(uid < mirror ? mirror - 1 - uid : uid) * kPlanInts;
 #pragma unroll
     for (int i = 0; i < kPlanInts; ++i) pu[i] = src[i];
   }
@@ -885,7 +890,7 @@ hipError_t launch(const AttnArgs& a, const Scalars& s, hipStream_t st) {
   int device = 0;
   const int32_t cus = hipGetDevice(&device) == hipSuccess ? slots_of(device) / 2 : 0;
   const int32_t slots = a.workspace != nullptr ? slots_of(device) : 0;
-  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0, 1};
+  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0, 1, 0};
   if (slots > 0 && a.workspace_bytes >= split_workspace_bytes(slots))
     split = round_split(static_cast<int32_t>(items), slots, (a.cur_len + kBN - 1) / kBN);
   AttnArgs b = a;
@@ -909,7 +914,18 @@ hipError_t launch(const AttnArgs& a, const Scalars& s, hipStream_t st) {
   }
   b.append_first = static_cast<int32_t>(blocks);
   const dim3 grid(static_cast<uint32_t>(blocks + copies));
-  const int32_t units = b.plan != nullptr ? static_cast<int32_t>(blocks) : 0;
+  // A plan with cut items that fills one round of more units than CUs:
+  // workgroups i and i + cus share a CU, and its two units end when their sum
+  // does.  In the plan's order (longest first) the longest would join the middle
+  // one and the middle the shortest, so the first half runs in reverse: the CU of
+  // its lightest unit takes the heaviest of the rest.  us, plan's order / so: 1024
+  // tokens, B=2, 16 heads, a tenth retained 41.1 / 39.7, two fifths 50.0 / 47.9,
+  // uneven heads 32.7 / 33.3; 1600 tokens, B=1 43.9 / 41.8, 62.5 / 58.0, 45.4 / 42.9;
+  // 576 tokens, B=3, 12 heads 23.3 / 21.7.  More than one round, and plans without cuts (dealt to
+  // XCDs by head), keep the plan's order.
+  int32_t units = b.plan != nullptr ? static_cast<int32_t>(blocks) : 0;
+  if (b.plan != nullptr && blocks > items && blocks > cus && blocks <= 2LL * cus && cus < 0x4000)
+    units = static_cast<int32_t>(0x80000000u | static_cast<uint32_t>(cus) << 16 | static_cast<uint32_t>(blocks));
   if (a.cur_len % kBN != 0 && a.cur_len < kMixedBelow)
     seg_attn_pipe_kernel<DT, DT, VDT, true><<<grid, 256, 0, st>>>(b.plan, units, b, s, n_qt, split);
   else

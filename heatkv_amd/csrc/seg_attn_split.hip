@@ -905,7 +905,7 @@ hipError_t launch_half(const AttnArgs& a, const Scalars& s, hipStream_t st, int3
   if (items > 0x3fffffffLL) return hipErrorInvalidConfiguration;
   int device = 0;
   const int32_t slots = a.workspace != nullptr && hipGetDevice(&device) == hipSuccess ? split_slots(device) : 0;
-  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0, 1};
+  RoundSplit split{static_cast<int32_t>(items), 0, 0, 0, 1, 0};
   if (slots > 0 && a.workspace_bytes >= split_workspace_bytes(slots))
     split = round_split(static_cast<int32_t>(items), slots, (a.cur_len + kBN - 1) / kBN);
   AttnArgs b = a;
