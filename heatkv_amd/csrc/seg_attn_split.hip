@@ -942,17 +942,22 @@ hipError_t launch_half(const AttnArgs& a, const Scalars& s, hipStream_t st, int3
 // halves / 8 waves at 144, 400, 576, 1024, 1600, 2304 tokens: planned 16.1 /
 // 19.5, 25.7 / 33.0, 30.7 / 39.9, 59.2 / 63.6, 105.0 / 107.1, 204 / 198; not
 // planned 17.2 / 20.4, 26.9 / 33.8, 37.0 / 47.2, 58.5 / 96.9, 105.7 / 126,
-// 203 / 229; not planned 4096 tokens 613 / 587).  So: up to one 256-query
-// item per CU (below two without a plan), or where half tiles save at least
-// an eighth of the padded queries (576 tokens, 768 items: 135 / 143 us; 1600
-// tokens save 7 %: 771 / 753).
+// 203 / 229; not planned 4096 tokens 613 / 587).  So, with a plan: up to one
+// 128-query workgroup per CU, and up to one 256-query item per CU from 2048
+// tokens (between the two some CUs share two halves while others have one:
+// 1024 tokens, B=3, 12 heads 61.6 / 59.4; 1008 tokens, 16 heads, a twentieth
+// retained 65.8 / 59.2; 1600 tokens, uneven heads 109.8 / 108.6; but 2304 tokens,
+// B=1 111.8 / 117.0); without one: below two 256-query items per CU.  And where
+// half tiles save at least an eighth of the padded queries (576 tokens, 768
+// items: 135 / 143 us; 1600 tokens save 7 %: 771 / 753).
 bool split_in_halves(const AttnArgs& a) {
   int device = 0;
   const int32_t cus = hipGetDevice(&device) == hipSuccess ? split_slots(device) / 2 : 0;
   const int64_t t256 = (static_cast<int64_t>(a.cur_len) + kSBM - 1) / kSBM;
   const int64_t t128 = (static_cast<int64_t>(a.cur_len) + 127) / 128;
   const int64_t items = static_cast<int64_t>(a.batch) * a.heads * t256;
-  if (a.plan != nullptr ? items <= cus : items < 2 * static_cast<int64_t>(cus)) return true;
+  const int64_t few = a.cur_len >= 2048 ? items : 2 * items;
+  if (a.plan != nullptr ? few <= cus : items < 2 * static_cast<int64_t>(cus)) return true;
   return 8 * t128 <= 7 * 2 * t256;
 }
 
