@@ -128,16 +128,20 @@ def load():
                 "`python heatkv_amd/csrc/build.py`"
             )
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
-            fn = getattr(lib, name)
-            fn.restype = res
-            fn.argtypes = args
-        have = int(lib.hkv_version())
+        rebuild = "rebuild it with `python heatkv_amd/csrc/build.py`"
+        version = getattr(lib, "hkv_version", None)
+        have = int(version()) if version is not None else 0
         if have != ABI_VERSION:
             raise RuntimeError(
                 f"{LIB_PATH} reports ABI version {have >> 16}.{(have >> 8) & 255}.{have & 255}; these "
-                f"bindings need {ABI_VERSION >> 16}.{(ABI_VERSION >> 8) & 255}.{ABI_VERSION & 255} -- rebuild it "
-                "with `python heatkv_amd/csrc/build.py`")
+                f"bindings need {ABI_VERSION >> 16}.{(ABI_VERSION >> 8) & 255}.{ABI_VERSION & 255} -- {rebuild}")
+        for name, (res, args) in SIGNATURES.items():
+            # an earlier build of the same version lacks the entry points added since
+            fn = getattr(lib, name, None)
+            if fn is None:
+                raise RuntimeError(f"{LIB_PATH} has no {name}: it is older than these bindings -- {rebuild}")
+            fn.restype = res
+            fn.argtypes = args
         _load_op_call(lib)
         _lib = lib
     return _lib

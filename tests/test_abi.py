@@ -144,3 +144,20 @@ def test_bind_refuses_small_or_unbound_blocks():
     blank = (ctypes.c_int64 * ((size + 7) // 8))()
     code = lib.hkv_segmented_attention_call(ctypes.addressof(blank), 1, 1, 1, 1, 1, 1, None)
     assert code == _lib.HKV_ERR_INVALID_ARG
+
+
+@pytest.mark.parametrize("source,missing", [("int hkv_version(void) { return 0x000300; }", "hkv_"),
+                                            ("int hkv_version(void) { return 0x000200; }", "ABI version 0.2.0"),
+                                            ("int hkv_something(void) { return 0; }", "ABI version 0.0.0")],
+                         ids=["same version, fewer entry points", "other version", "no version"])
+def test_an_older_library_is_refused_with_the_way_out(source, missing, tmp_path, monkeypatch):
+    """A library that lacks entry points, whatever version it reports, is
+    refused with the command that rebuilds it."""
+    (tmp_path / "old.c").write_text(source + "\n")
+    path = str(tmp_path / "libold.so")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", path], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", path)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(RuntimeError, match="rebuild it with") as e:
+        _lib.load()
+    assert missing in str(e.value)
