@@ -168,6 +168,12 @@ def _load_op_call(lib) -> None:
         return
     names = ("hkv_segmented_attention", "hkv_segmented_attention_split", "hkv_segmented_attention_split_bytes",
              "hkv_segmented_attention_item_shape", "hkv_qkv_produce", "hkv_pack_segments")
+    # the extension calls plain addresses: it must have been compiled for these prototypes
+    code = {_c_i32: "i", _c_i64: "l", ctypes.c_float: "f", _c_p: "p"}
+    want = tuple("".join(code[t] for t in (SIGNATURES[n][0], *SIGNATURES[n][1])) for n in names)
+    if getattr(_op_call, "prototypes", tuple)() != want:
+        raise RuntimeError("heatkv_amd/_op_call.so was built for other entry points than these bindings'; rebuild it "
+                           "with `python heatkv_amd/csrc/build.py`")
     _op_call.init(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), _ENV_DATA,
                   tuple(os.environ.encodekey(n) for n in _OP_KNOBS), _workspaces, _device_ok)
     op_call = _op_call

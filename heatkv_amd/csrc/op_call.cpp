@@ -28,6 +28,8 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cstring>
+#include <string>
+#include <type_traits>
 
 #include "heatkv.h"
 
@@ -369,6 +371,27 @@ PyObject* guarded(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
 }
 
+// A prototype as compiled here: return and argument types, i int32, l int64,
+// f float, p pointer.
+template <typename T>
+constexpr char type_code() {
+  if (std::is_pointer<T>::value) return 'p';
+  if (std::is_same<T, float>::value) return 'f';
+  return sizeof(T) == 8 ? 'l' : 'i';
+}
+template <typename R, typename... A>
+std::string prototype(R (*)(A...)) {
+  return {type_code<R>(), type_code<A>()...};
+}
+
+// prototypes(): those of init's entry points, in its order.
+PyObject* prototypes(PyObject*, PyObject*) {
+  const std::string p[6] = {prototype(g.attention), prototype(g.attention_split), prototype(g.split_bytes),
+                            prototype(g.item_shape), prototype(g.produce), prototype(g.pack)};
+  return Py_BuildValue("(ssssss)", p[0].c_str(), p[1].c_str(), p[2].c_str(), p[3].c_str(), p[4].c_str(),
+                       p[5].c_str());
+}
+
 // init(addresses, env, knobs, workspaces, devices)
 PyObject* init(PyObject*, PyObject* args) {
   unsigned long long a[6];
@@ -402,6 +425,7 @@ PyMethodDef methods[] = {
      "The QKV producer's launch, or None"},
     {"pack", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(guarded<pack_call>)), METH_FASTCALL,
      "The slab pack's launch, or None"},
+    {"prototypes", prototypes, METH_NOARGS, "The entry points' prototypes as compiled, in init's order"},
     {"init", init, METH_VARARGS, "init(addresses, env, knobs, workspaces, devices)"},
     {nullptr, nullptr, 0, nullptr}};
 

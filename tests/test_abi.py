@@ -161,3 +161,26 @@ def test_an_older_library_is_refused_with_the_way_out(source, missing, tmp_path,
     with pytest.raises(RuntimeError, match="rebuild it with") as e:
         _lib.load()
     assert missing in str(e.value)
+
+
+@pytest.mark.parametrize("stale", ["without prototypes", "other prototypes"])
+def test_an_extension_built_for_other_entry_points_is_refused(stale, monkeypatch):
+    """The extension calls the library through plain addresses, so one whose
+    compiled prototypes are not the bindings' must not be given any."""
+    import sys
+    import types
+
+    import heatkv_amd
+
+    given = []
+    fake = types.ModuleType("heatkv_amd._op_call")
+    fake.init = lambda *a: given.append(a)
+    if stale == "other prototypes":
+        fake.prototypes = lambda: ("i",) * 6
+    lib = _lib.load()
+    monkeypatch.setitem(sys.modules, "heatkv_amd._op_call", fake)
+    monkeypatch.setattr(heatkv_amd, "_op_call", fake, raising=False)
+    monkeypatch.setattr(_lib, "op_call", None)
+    with pytest.raises(RuntimeError, match="rebuild it with"):
+        _lib._load_op_call(lib)
+    assert not given and _lib.op_call is None
