@@ -12,6 +12,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 
 import torch
 
@@ -157,13 +158,16 @@ def _load_op_call(lib) -> None:
     """Imports the extension and gives it the library's entry points and the
     dicts it looks into: the environment (with any of ``_OP_KNOBS`` set, calls
     take the operators' Python bodies), the per-stream workspaces and the
-    checked devices."""
+    checked devices.  Without it (not built, or built for another torch or
+    another header) the Python bodies take every call: the same launches at a
+    few us more of host time each, and a warning."""
     global op_call
+    rebuild = "the operators run their Python bodies; rebuild it with `python heatkv_amd/csrc/build.py`"
     try:
         from . import _op_call
     except ImportError as e:
-        raise RuntimeError(f"the native call path heatkv_amd/_op_call.so cannot be loaded ({e}); build it with "
-                           "`python heatkv_amd/csrc/build.py`") from e
+        warnings.warn(f"heatkv_amd/_op_call.so cannot be loaded ({e}): {rebuild}", RuntimeWarning, stacklevel=3)
+        return
     if not isinstance(_ENV_DATA, dict):  # pragma: no cover - another platform's os.environ
         return
     names = ("hkv_segmented_attention", "hkv_segmented_attention_split", "hkv_segmented_attention_split_bytes",
@@ -172,8 +176,9 @@ def _load_op_call(lib) -> None:
     code = {_c_i32: "i", _c_i64: "l", ctypes.c_float: "f", _c_p: "p"}
     want = tuple("".join(code[t] for t in (SIGNATURES[n][0], *SIGNATURES[n][1])) for n in names)
     if getattr(_op_call, "prototypes", tuple)() != want:
-        raise RuntimeError("heatkv_amd/_op_call.so was built for other entry points than these bindings'; rebuild it "
-                           "with `python heatkv_amd/csrc/build.py`")
+        warnings.warn(f"heatkv_amd/_op_call.so was built for other entry points than these bindings': {rebuild}",
+                      RuntimeWarning, stacklevel=3)
+        return
     _op_call.init(tuple(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names), _ENV_DATA,
                   tuple(os.environ.encodekey(n) for n in _OP_KNOBS), _workspaces, _device_ok)
     op_call = _op_call

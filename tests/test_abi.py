@@ -181,6 +181,23 @@ def test_an_extension_built_for_other_entry_points_is_refused(stale, monkeypatch
     monkeypatch.setitem(sys.modules, "heatkv_amd._op_call", fake)
     monkeypatch.setattr(heatkv_amd, "_op_call", fake, raising=False)
     monkeypatch.setattr(_lib, "op_call", None)
-    with pytest.raises(RuntimeError, match="rebuild it with"):
+    with pytest.warns(RuntimeWarning, match="rebuild it with"):
         _lib._load_op_call(lib)
     assert not given and _lib.op_call is None
+
+
+def test_the_library_loads_without_the_extension(monkeypatch):
+    """The extension only shortens the host's part of a call: without it the
+    library loads (with a warning) and the Python bodies take the calls."""
+    import sys
+
+    import heatkv_amd
+
+    _lib.load()
+    monkeypatch.delattr(heatkv_amd, "_op_call", raising=False)
+    monkeypatch.setitem(sys.modules, "heatkv_amd._op_call", None)  # import fails
+    monkeypatch.setattr(_lib, "op_call", None)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.warns(RuntimeWarning, match="rebuild it with"):
+        lib = _lib.load()
+    assert lib.hkv_version() == _lib.ABI_VERSION and _lib.op_call is None
