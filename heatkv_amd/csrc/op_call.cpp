@@ -27,6 +27,7 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <type_traits>
@@ -149,6 +150,20 @@ bool plan_fits(PyObject* plan, int32_t queries, int64_t B, int64_t L, int dev, c
          whole(PyTuple_GET_ITEM(shape.p, 0), &b) && whole(PyTuple_GET_ITEM(shape.p, 1), &l) && b == B && l == L;
 }
 
+// Where an all-fp32 call is better split (_split_values_pays in
+// real_pruning_fused_attention.py, which holds the figures; `split_from` and
+// `split_slab` are its two limits).
+bool split_values_pays(int64_t B, int64_t H, int64_t L, int64_t cap, int64_t split_from, int64_t split_slab, int dev) {
+  const int64_t pairs = B * H, rows = pairs * L;
+  int64_t limit = split_slab;
+  if (rows >= split_from) limit = std::max((L > 256 ? 8 : 4) * rows, split_slab / 4);
+  if (B * cap > limit) return false;
+  if (rows < 8192 || pairs <= 64) return true;
+  int32_t cus = 0;  // the staged kernel's resident workgroups
+  if (g.item_shape(HKV_DTYPE_F32, HKV_DTYPE_F32, HKV_DTYPE_F32, 1, 0, 0, dev, &cus) < 0) return false;
+  return pairs * ((L + 127) / 128) > cus;
+}
+
 // attention(q, persisted_k, persisted_v, segment_starts, segment_ends,
 // segment_counts, current_k, current_v, softmax_scale, softmax_mode,
 // return_lse, out_dtype, work_plan, k_split_rows, split_values_rows,
@@ -200,7 +215,8 @@ PyObject* attention_call(PyObject* const* args, Py_ssize_t n) {
   // call itself unless the caller has them
   const bool rows32 = qc == HKV_DTYPE_F32 && vc != HKV_DTYPE_F32;
   if (k_split && !rows32) Py_RETURN_NONE;
-  const bool split_v = qc == HKV_DTYPE_F32 && vc == HKV_DTYPE_F32 && (B * H * L >= split_from || B * cap <= split_slab);
+  const bool split_v =
+      qc == HKV_DTYPE_F32 && vc == HKV_DTYPE_F32 && split_values_pays(B, H, L, cap, split_from, split_slab, dev);
   const bool splits = (rows32 && !k_split) || split_v;
   if (splits && (!aligned(ck) || !aligned(pk) || (split_v && (!aligned(cv) || !aligned(pv))))) Py_RETURN_NONE;
   const int32_t queries = rows32 ? g.item_shape(qc, HKV_DTYPE_SPLIT_ROWS, vc, 1, 0, 0, 0, nullptr) : 128;

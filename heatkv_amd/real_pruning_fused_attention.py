@@ -145,27 +145,53 @@ def _split_rows_path(q_dtype, k_dtype, v_dtype, qk_mode: int, value_mode: int) -
             and qk_mode != 2 and value_mode != 2)
 
 
-# All-fp32 calls split K and V ahead of the attention: faster than the staged
-# kernel at every size (one image pair, 16 heads, a tenth retained, whole calls,
-# us, split / staged: 4 tokens 10.4 / 16.0, 36: 13.3 / 16.4, 64: 15.3 / 16.2; one
-# image, 5 heads 144: 19.7 / 27.7, 400: 30.9 / 48.0; 2304 tokens, one pair: 305 /
-# 538).  The copies hold a row for every slab row, so where the slab is large
-# (64 MB of copies) and the call small (fewer current rows, batch x heads x
-# length, than this), the staged kernel's call without them stays.
+# All-fp32 calls split K and V ahead of the attention where that pays: the copies
+# cost ~0.7 ns a current row and ~0.03 ns a slab row (kept or not: their blocks
+# look for the kept ones), and a byte of scratch for each byte of K and V, the
+# slab's included.  Whole calls, planned with the append, us, split / staged
+# kernel, by batch x heads:
+# * slab rows against current rows.  Fewer than _SPLIT_VALUES_ROWS current rows:
+#   the launch latency decides, and up to _SPLIT_VALUES_SLAB_ROWS slab rows the
+#   split wins (4x32, 4 tokens: 40k slab rows 14.1 / 18.4, 200k 18.5 / 18.5, 800k
+#   36.3 / 18.5).  From there on up to 4 slab rows per current row (4x16, 144
+#   tokens: 4.5 29.6 / 31.9, 22 33.8 / 32.1), and 8 above 256 tokens, where every
+#   row is read by more query tiles (4x16, 300 tokens: 2.2 39.6 / 44.6, 10.6 44.6 /
+#   44.5; 8x32, 400: 4 161 / 210, 16 197 / 210).
+# * a launch that the staged kernel runs in one round of its workgroups (one per
+#   CU) has nothing to gain but latency, which _SPLIT_ROUND_ROWS rows use up
+#   (8x32: 24 tokens 18.0 / 20.7, 36 21.8 / 21.0, 64 28.5 / 24.5, 128 39.5 / 34.0,
+#   but 144, in two rounds, 49.2 / 63.5; 4x32: 64 tokens 23.4 / 20.7, 256 46.0 /
+#   43.3), except with few and then longer (batch, head) pairs (4x16: 128 tokens
+#   26.2 / 25.9, 200 33.4 / 38.1, 400 48.1 / 57.4).
 _SPLIT_VALUES_ROWS = 4096
 _SPLIT_VALUES_SLAB_ROWS = 65536
+_SPLIT_ROUND_ROWS = 8192
+_SPLIT_ROUND_PAIRS = 64
+
+
+def _split_values_pays(batch: int, heads: int, length: int, capacity: int, cus) -> bool:
+    """The rule above; ``cus()``: workgroups of the staged kernel in one round.
+    The native call path (csrc/op_call.cpp) follows the same rule."""
+    pairs = batch * heads
+    rows = pairs * length
+    if rows < _SPLIT_VALUES_ROWS:
+        limit = _SPLIT_VALUES_SLAB_ROWS
+    else:
+        limit = max((8 if length > 256 else 4) * rows, _SPLIT_VALUES_SLAB_ROWS // 4)
+    if batch * capacity > limit:
+        return False
+    return rows < _SPLIT_ROUND_ROWS or pairs <= _SPLIT_ROUND_PAIRS or pairs * (-(-length // 128)) > cus()
 
 
 def _split_values_path(q, k, v, slab_k, qk_mode: int, value_mode: int) -> bool:
     """fp32 q, k and v at the default (or tf32) dot modes run the split-row
-    kernel's 128-query form on split copies of K and V; otherwise (and for small
-    calls on very large slabs, and with HKV_ATTN_SPLIT_ROWS=0) the
-    register-staged kernel, which splits every tile for every query tile itself."""
+    kernel's 128-query form on split copies of K and V where the copies pay
+    (and HKV_ATTN_SPLIT_ROWS is not 0); otherwise the register-staged kernel,
+    which splits every tile for every query tile itself."""
     return (q.dtype == torch.float32 and k.dtype == torch.float32 and v.dtype == torch.float32
-            and qk_mode != 2 and value_mode != 2
-            and (q.shape[0] * q.shape[1] * q.shape[2] >= _SPLIT_VALUES_ROWS
-                 or slab_k.shape[0] * slab_k.shape[1] <= _SPLIT_VALUES_SLAB_ROWS)
-            and _split_rows_enabled())
+            and qk_mode != 2 and value_mode != 2 and _split_rows_enabled()
+            and _split_values_pays(q.shape[0], q.shape[1], q.shape[2], slab_k.shape[1],
+                                   lambda: attention_item_shape(q.dtype, k.dtype, v.dtype, device=q.device)[1]))
 
 
 def split_rows_k_format(q_dtype, k_dtype, v_dtype) -> bool:

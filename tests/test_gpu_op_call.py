@@ -110,6 +110,43 @@ def test_attention_taken(device, dtypes, kw, planned):
         assert same(got, body(fused_real_pruning_flat_segmented_attention, **big)) and not same(got, want)
 
 
+@pytest.mark.parametrize("B,H,L,cap,split", [
+    (1, 2, 16, 65536, True), (1, 2, 16, 65537, False),         # few rows: the slab's own limit
+    (4, 16, 64, 4096, True), (4, 16, 64, 4097, False),         # 4096 rows: 4 slab rows each
+    (1, 16, 256, 16384, True), (1, 16, 256, 16385, False),
+    (1, 16, 257, 32896, True), (1, 16, 257, 32897, False),     # 8 above 256 tokens
+    (8, 32, 16, 25000, False),                                 # rows a pool of kept slabs would have
+    (5, 13, 126, 8, True), (5, 13, 127, 8, False),             # one round of the staged kernel
+    (4, 16, 128, 8, True), (8, 32, 128, 8, False), (8, 33, 128, 8, True), (8, 32, 129, 8, True)])
+def test_fp32_split_copies_only_where_they_pay(device, B, H, L, cap, split, monkeypatch):
+    """All-fp32 calls make split copies on the inner side of each limit and run
+    as they are, in no more memory than their outputs, on the other: both
+    paths of the operator alike."""
+    g = torch.Generator(device=device).manual_seed(3)
+    rand = lambda *s: torch.randn(s, generator=g, device=device)  # noqa: E731
+    table = torch.zeros((H, 1), dtype=torch.int32, device=device)
+    a = dict(q=rand(B, H, L, D), persisted_k=rand(B, cap, D), persisted_v=rand(B, cap, D), segment_starts=table,
+             segment_ends=table + min(cap, 8), segment_counts=torch.ones(H, dtype=torch.int32, device=device),
+             current_k=rand(B, H, L, D), current_v=rand(B, H, L, D), softmax_scale=0.09)
+
+    def measured(fn):
+        torch.cuda.synchronize(device)
+        torch.cuda.reset_peak_memory_stats(device)
+        before = torch.cuda.memory_allocated(device)
+        out = fn()
+        torch.cuda.synchronize(device)
+        return out, torch.cuda.max_memory_allocated(device) - before - out.numel() * out.element_size()
+
+    got, used = measured(lambda: native(a))
+    want, body_used = measured(lambda: body(fused_real_pruning_flat_segmented_attention, **a))
+    monkeypatch.setenv("HKV_ATTN_SPLIT_ROWS", "0")
+    staged, _ = measured(lambda: fused_real_pruning_flat_segmented_attention(**a))
+    assert same(got, want) and same(got, staged) != split
+    copies = 2 * 512 * B * (cap + H * L)
+    for n in (used, body_used):
+        assert (n >= copies) if split else (n < 4096)
+
+
 def _changes(device):
     """Calls outside the native path, or refused: name -> changed arguments."""
     a = attention_args(device)
