@@ -637,9 +637,22 @@ def fused_real_pruning_flat_segmented_attention(
     # fp32 K (and V) rows go to the split-row kernels as split copies made by
     # the same call (the q split happens in the kernel)
     splits = (split and not k_split_rows) or split_v
-    converted = promoted or splits
     lib = _lib.load()
     scratch = None
+    no_room = False
+    if splits:
+        need = int(lib.hkv_segmented_attention_split_bytes(batch_size, num_heads, current_len,
+                                                           int(persisted_k.shape[1]),
+                                                           _lib.dtype_code(current_v.dtype)))
+        _lib.check(min(need, 0))
+        try:
+            scratch = torch.empty((need,), device=q.device, dtype=torch.uint8)
+        except torch.OutOfMemoryError:
+            if not split_v:
+                raise
+            # no room for the copies: the staged kernel takes the fp32 rows as they are
+            splits, no_room = False, True
+    converted = promoted or splits or no_room
     if splits:
         # the split reads 16 bytes per access (a slab that the append writes
         # stays itself: the library refuses it when it is not aligned)
@@ -648,11 +661,6 @@ def fused_real_pruning_flat_segmented_attention(
         if split_v:
             current_v = _aligned(current_v)
             persisted_v = persisted_v if append_offsets is not None else _aligned(persisted_v)
-        need = int(lib.hkv_segmented_attention_split_bytes(batch_size, num_heads, current_len,
-                                                           int(persisted_k.shape[1]),
-                                                           _lib.dtype_code(current_v.dtype)))
-        _lib.check(min(need, 0))
-        scratch = torch.empty((need,), device=q.device, dtype=torch.uint8)
     args = [
         q.data_ptr(), persisted_k.data_ptr(), persisted_v.data_ptr(),
         segment_starts.data_ptr(), segment_ends.data_ptr(), segment_counts.data_ptr(),

@@ -147,6 +147,30 @@ def test_fp32_split_copies_only_where_they_pay(device, B, H, L, cap, split, monk
         assert (n >= copies) if split else (n < 4096)
 
 
+def test_fp32_call_without_room_for_split_copies(device, monkeypatch):
+    """Where the split copies cannot be allocated the call runs as it does
+    without them."""
+    a = attention_args(device, (F32, F32, F32), L=300)
+    for n in ("persisted_k", "persisted_v"):
+        a[n] = torch.cat((a[n], a[n].new_zeros(2, 30000, D)), dim=1)
+    fn = fused_real_pruning_flat_segmented_attention
+    with monkeypatch.context() as m:
+        m.setenv("HKV_ATTN_SPLIT_ROWS", "0")
+        want = fn(**a)
+    assert not same(fn(**a), want)  # split where there is room
+    torch.cuda.synchronize(device)
+    torch.cuda.empty_cache()
+    room = torch.cuda.memory_reserved(device) + (24 << 20)  # the output fits, 64 MB of copies do not
+    try:
+        torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(device).total_memory, device)
+        for call in (fn, lambda **kw: body(fn, **kw)):
+            got = call(**a)
+            torch.cuda.synchronize(device)
+            assert same(got, want)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, device)
+
+
 def _changes(device):
     """Calls outside the native path, or refused: name -> changed arguments."""
     a = attention_args(device)
