@@ -373,6 +373,69 @@ int64_t hkv_segmented_attention_split_bytes(int32_t batch, int32_t heads, int32_
   return rows * 512 * (v_dtype == HKV_DTYPE_F32 ? 2 : 1);
 }
 
+// The split call on validated arguments `a` (fp32 rows).
+namespace {
+int32_t launch_split_call(const hkv::AttnArgs& a, void* scratch, int64_t scratch_bytes, void* stream) {
+  const bool with_v = a.v_dtype == HKV_DTYPE_F32;
+  if (a.q_dtype != HKV_DTYPE_F32 || a.k_dtype != HKV_DTYPE_F32 || a.qk_dot_mode == 2 || a.value_dot_mode == 2)
+    return fail(HKV_ERR_UNSUPPORTED,
+                "the split call takes float32 q and k and the default (or tf32) dot modes (got q %d, k %d, modes "
+                "%d/%d)", a.q_dtype, a.k_dtype, a.qk_dot_mode, a.value_dot_mode);
+  // the split reads its rows 16 bytes per access
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(a.slab_k) | reinterpret_cast<uintptr_t>(a.cur_k) |
+                         (with_v ? reinterpret_cast<uintptr_t>(a.slab_v) | reinterpret_cast<uintptr_t>(a.cur_v) : 0) |
+                         reinterpret_cast<uintptr_t>(scratch);
+  if ((bits & 15) != 0) return fail(HKV_ERR_INVALID_ARG, "the split needs 16-byte aligned fp32 tensors and scratch");
+  const int64_t need =
+      hkv_segmented_attention_split_bytes(a.batch, a.heads, a.cur_len, a.slab_capacity, a.v_dtype);
+  if (!scratch || scratch_bytes < need)
+    return fail(HKV_ERR_INVALID_ARG, "scratch of %lld bytes is smaller than the %lld required",
+                static_cast<long long>(scratch ? scratch_bytes : 0), static_cast<long long>(need));
+  const int64_t slab_bytes = static_cast<int64_t>(a.batch) * a.slab_capacity * 512;
+  const int64_t cur_rows = static_cast<int64_t>(a.batch) * a.heads * a.cur_len;
+  uint8_t* const s = static_cast<uint8_t*>(scratch);
+  hkv::SplitOperands o{};
+  o.slab_k = static_cast<const float*>(a.slab_k);
+  o.cur_k = static_cast<const float*>(a.cur_k);
+  o.cur_k_out = s;
+  o.slab_k_out = s + cur_rows * 512;
+  if (with_v) {
+    o.slab_v = static_cast<const float*>(a.slab_v);
+    o.cur_v = static_cast<const float*>(a.cur_v);
+    o.cur_v_out = o.slab_k_out + slab_bytes;
+    o.slab_v_out = o.cur_v_out + cur_rows * 512;
+  }
+  o.seg_starts = a.seg_starts;
+  o.seg_ends = a.seg_ends;
+  o.seg_counts = a.seg_counts;
+  o.slab_capacity = a.slab_capacity;
+  o.cur_rows = cur_rows;
+  o.batch = a.batch;
+  o.heads = a.heads;
+  o.max_segments = a.max_segments;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  hipError_t e = hkv::launch_split_operands(o, with_v, st);
+  if (e == hipSuccess) {
+    hkv::AttnArgs b = a;
+    b.slab_k = o.slab_k_out;
+    b.cur_k = o.cur_k_out;
+    b.k_dtype = hkv::kSplitRows;
+    if (with_v) {
+      b.slab_v = o.slab_v_out;
+      b.cur_v = o.cur_v_out;
+      b.v_dtype = hkv::kSplitRows;
+    }
+    b.append_offsets = nullptr;
+    b.append2_offsets = nullptr;
+    e = hkv::launch_segmented_attention(b, st);
+  }
+  if (e == hipSuccess && a.append_offsets != nullptr) e = hkv::launch_append(a, st);
+  if (e != hipSuccess)
+    return fail(HKV_ERR_LAUNCH, "segmented attention launch failed: %s", hipGetErrorString(e));
+  return ok();
+}
+}  // namespace
+
 int32_t hkv_segmented_attention_split(const void* q, void* slab_k, void* slab_v, const int32_t* seg_starts,
                                       const int32_t* seg_ends, const int32_t* seg_counts, const void* cur_k,
                                       const void* cur_v, void* out, float* lse, int32_t batch, int32_t heads,
@@ -391,62 +454,7 @@ int32_t hkv_segmented_attention_split(const void* q, void* slab_k, void* slab_v,
       qk_dot_mode, value_dot_mode, work_plan, plan_units, workspace, workspace_bytes, append_offsets, slab2_k,
       slab2_v, slab2_capacity, append2_offsets);
   if (code != 0) return code;
-  const bool with_v = v_dtype == HKV_DTYPE_F32;
-  if (q_dtype != HKV_DTYPE_F32 || k_dtype != HKV_DTYPE_F32 || qk_dot_mode == 2 || value_dot_mode == 2)
-    return fail(HKV_ERR_UNSUPPORTED,
-                "the split call takes float32 q and k and the default (or tf32) dot modes (got q %d, k %d, modes "
-                "%d/%d)", q_dtype, k_dtype, qk_dot_mode, value_dot_mode);
-  // the split reads its rows 16 bytes per access
-  const uintptr_t bits = reinterpret_cast<uintptr_t>(slab_k) | reinterpret_cast<uintptr_t>(cur_k) |
-                         (with_v ? reinterpret_cast<uintptr_t>(slab_v) | reinterpret_cast<uintptr_t>(cur_v) : 0) |
-                         reinterpret_cast<uintptr_t>(scratch);
-  if ((bits & 15) != 0) return fail(HKV_ERR_INVALID_ARG, "the split needs 16-byte aligned fp32 tensors and scratch");
-  const int64_t need = hkv_segmented_attention_split_bytes(batch, heads, cur_len, slab_capacity, v_dtype);
-  if (!scratch || scratch_bytes < need)
-    return fail(HKV_ERR_INVALID_ARG, "scratch of %lld bytes is smaller than the %lld required",
-                static_cast<long long>(scratch ? scratch_bytes : 0), static_cast<long long>(need));
-  const int64_t slab_bytes = static_cast<int64_t>(batch) * slab_capacity * 512;
-  const int64_t cur_rows = static_cast<int64_t>(batch) * heads * cur_len;
-  uint8_t* const s = static_cast<uint8_t*>(scratch);
-  hkv::SplitOperands o{};
-  o.slab_k = static_cast<const float*>(slab_k);
-  o.cur_k = static_cast<const float*>(cur_k);
-  o.cur_k_out = s;
-  o.slab_k_out = s + cur_rows * 512;
-  if (with_v) {
-    o.slab_v = static_cast<const float*>(slab_v);
-    o.cur_v = static_cast<const float*>(cur_v);
-    o.cur_v_out = o.slab_k_out + slab_bytes;
-    o.slab_v_out = o.cur_v_out + cur_rows * 512;
-  }
-  o.seg_starts = seg_starts;
-  o.seg_ends = seg_ends;
-  o.seg_counts = seg_counts;
-  o.slab_capacity = slab_capacity;
-  o.cur_rows = cur_rows;
-  o.batch = batch;
-  o.heads = heads;
-  o.max_segments = max_segments;
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  hipError_t e = hkv::launch_split_operands(o, with_v, st);
-  if (e == hipSuccess) {
-    hkv::AttnArgs b = a;
-    b.slab_k = o.slab_k_out;
-    b.cur_k = o.cur_k_out;
-    b.k_dtype = hkv::kSplitRows;
-    if (with_v) {
-      b.slab_v = o.slab_v_out;
-      b.cur_v = o.cur_v_out;
-      b.v_dtype = hkv::kSplitRows;
-    }
-    b.append_offsets = nullptr;
-    b.append2_offsets = nullptr;
-    e = hkv::launch_segmented_attention(b, st);
-  }
-  if (e == hipSuccess && append_offsets != nullptr) e = hkv::launch_append(a, st);
-  if (e != hipSuccess)
-    return fail(HKV_ERR_LAUNCH, "segmented attention launch failed: %s", hipGetErrorString(e));
-  return ok();
+  return launch_split_call(a, scratch, scratch_bytes, stream);
 }
 
 // The argument block of hkv_segmented_attention_bind: the validated launch
@@ -516,8 +524,10 @@ int32_t hkv_segmented_attention_bind2(void* bound, int64_t bound_bytes, const in
   return ok();
 }
 
-int32_t hkv_segmented_attention_call(const void* bound, const void* q, void* slab_k, void* slab_v,
-                                     const void* cur_k, const void* cur_v, void* out, void* stream) {
+// `a`: the bound arguments with this call's tensors (0 or an error code).
+namespace {
+int32_t bound_args(hkv::AttnArgs& a, const void* bound, const void* q, void* slab_k, void* slab_v, const void* cur_k,
+                   const void* cur_v, void* out) {
   const BoundAttention* b = static_cast<const BoundAttention*>(bound);
   if (b == nullptr || b->tag != kBoundTag) return fail(HKV_ERR_INVALID_ARG, "not a bound attention call");
   if (!q || !cur_k || !cur_v || !out || (b->a.slab_capacity > 0 && (!slab_k || !slab_v)))
@@ -526,17 +536,35 @@ int32_t hkv_segmented_attention_call(const void* bound, const void* q, void* sla
       ((reinterpret_cast<uintptr_t>(slab_k) | reinterpret_cast<uintptr_t>(slab_v) |
         reinterpret_cast<uintptr_t>(cur_k) | reinterpret_cast<uintptr_t>(cur_v)) & 15) != 0)
     return fail(HKV_ERR_INVALID_ARG, "the append needs 16-byte aligned slab and current tensors");
-  hkv::AttnArgs a = b->a;
+  a = b->a;
   a.q = q;
   a.slab_k = slab_k;
   a.slab_v = slab_v;
   a.cur_k = cur_k;
   a.cur_v = cur_v;
   a.out = out;
+  return 0;
+}
+}  // namespace
+
+int32_t hkv_segmented_attention_call(const void* bound, const void* q, void* slab_k, void* slab_v,
+                                     const void* cur_k, const void* cur_v, void* out, void* stream) {
+  hkv::AttnArgs a;
+  const int32_t code = bound_args(a, bound, q, slab_k, slab_v, cur_k, cur_v, out);
+  if (code != 0) return code;
   const hipError_t e = hkv::launch_segmented_attention(a, static_cast<hipStream_t>(stream));
   if (e != hipSuccess)
     return fail(HKV_ERR_LAUNCH, "segmented attention launch failed: %s", hipGetErrorString(e));
   return ok();
+}
+
+int32_t hkv_segmented_attention_call_split(const void* bound, const void* q, void* slab_k, void* slab_v,
+                                           const void* cur_k, const void* cur_v, void* out, void* scratch,
+                                           int64_t scratch_bytes, void* stream) {
+  hkv::AttnArgs a;
+  const int32_t code = bound_args(a, bound, q, slab_k, slab_v, cur_k, cur_v, out);
+  if (code != 0) return code;
+  return launch_split_call(a, scratch, scratch_bytes, stream);
 }
 
 int32_t hkv_qkv_produce(const void* qkv, int64_t token_stride, const float* q_bias,

@@ -652,7 +652,7 @@ def fused_real_pruning_flat_segmented_attention(
                 raise
             # no room for the copies: the staged kernel takes the fp32 rows as they are
             splits, no_room = False, True
-    converted = promoted or splits or no_room
+    converted = promoted or (splits and not split_v) or no_room
     if splits:
         # the split reads 16 bytes per access (a slab that the append writes
         # stays itself: the library refuses it when it is not aligned)
@@ -674,30 +674,27 @@ def fused_real_pruning_flat_segmented_attention(
         int(work_plan.shape[0]) if work_plan is not None else 0,
         ws.data_ptr() if ws is not None else None, int(ws.numel()) if ws is not None else 0,
     ]
+    slab2 = (None, None, 0, None) if append_also is None else (
+        slab2_k.data_ptr(), slab2_v.data_ptr(), int(slab2_k.shape[1]), offsets2.data_ptr())
+    append = append_offsets.data_ptr() if append_offsets is not None else None
     if splits:
-        fn = lib.hkv_segmented_attention_split
-        args.append(append_offsets.data_ptr() if append_offsets is not None else None)
-        args += ([None, None, 0, None] if append_also is None else
-                 [slab2_k.data_ptr(), slab2_v.data_ptr(), int(slab2_k.shape[1]), offsets2.data_ptr()])
-        args += [scratch.data_ptr(), int(scratch.numel())]
+        fn, tail = lib.hkv_segmented_attention_split, (append, *slab2, scratch.data_ptr(), int(scratch.numel()))
     elif append_offsets is None:
-        fn = lib.hkv_segmented_attention
+        fn, tail = lib.hkv_segmented_attention, ()
     elif append_also is None:
-        fn = lib.hkv_segmented_attention_append
-        args.append(append_offsets.data_ptr())
+        fn, tail = lib.hkv_segmented_attention_append, (append,)
     else:
-        fn = lib.hkv_segmented_attention_append2
-        args += [append_offsets.data_ptr(), slab2_k.data_ptr(), slab2_v.data_ptr(), int(slab2_k.shape[1]),
-                 offsets2.data_ptr()]
-    args.append(stream.cuda_stream)
-    _lib.check(fn(*args))
+        fn, tail = lib.hkv_segmented_attention_append2, (append, *slab2)
+    _lib.check(fn(*args, *tail, stream.cuda_stream))
     if _bind is not None:
         # what a pre-bound call needs to repeat this launch for new q / k / v
         # / slab tensors of the same shapes (None when this call converted its
-        # inputs: those copies are per call)
+        # inputs otherwise than by the split call: those copies are per call)
         keep = (q, persisted_k, persisted_v, current_k, current_v, segment_starts, segment_ends, segment_counts,
                 work_plan, append_offsets, ws, append_also)
-        _bind.append(None if converted or lse is not None else (fn, args, output.shape, out_dtype, keep))
+        _bind.append(None if converted or lse is not None else
+                     (args, append, slab2, stream.cuda_stream, int(scratch.numel()) if splits else 0, output.shape,
+                      out_dtype, keep))
     if return_lse:
         return output, lse
     return output
@@ -718,31 +715,29 @@ class BoundSegmentedAttention:
     calls the operator."""
 
     __slots__ = ("_block", "_addr", "_call", "_out_shape", "_out_dtype", "_keep", "_dev", "_device", "_stream",
-                 "_qs", "_ps", "_qdt", "_kdt", "_vdt", "_skdt", "_svdt")
+                 "_qs", "_ps", "_qdt", "_kdt", "_vdt", "_skdt", "_svdt", "_scratch")
 
     def __init__(self, record, *, q, current_k, current_v, persisted_k, persisted_v):
-        fn, a, out_shape, out_dtype, keep = record
+        a, append, slab2, stream, scratch, out_shape, out_dtype, keep = record
         lib = _lib.load()
         size = int(lib.hkv_segmented_attention_bound_bytes())
         self._block = (ctypes.c_int64 * ((size + 7) // 8))()
         self._addr = ctypes.addressof(self._block)
-        append = a[28] if len(a) > 29 else None
-        if len(a) > 30:
+        bound = (self._addr, size, a[3], a[4], a[5], *a[10:28], append)
+        if slab2[3] is not None:
             # the second append destination (slab2 K/V, capacity, offsets) is bound with the rest
-            _lib.check(lib.hkv_segmented_attention_bind2(
-                self._addr, size, a[3], a[4], a[5], a[10], a[11], a[12], a[13], a[14], a[15], a[16], a[17], a[18],
-                a[19], a[20], a[21], a[22], a[23], a[24], a[25], a[26], a[27], append, a[29], a[30], a[31], a[32]))
+            _lib.check(lib.hkv_segmented_attention_bind2(*bound, *slab2))
         else:
-            _lib.check(lib.hkv_segmented_attention_bind(
-                self._addr, size, a[3], a[4], a[5], a[10], a[11], a[12], a[13], a[14], a[15], a[16], a[17], a[18],
-                a[19], a[20], a[21], a[22], a[23], a[24], a[25], a[26], a[27], append))
-        self._call = lib.hkv_segmented_attention_call
+            _lib.check(lib.hkv_segmented_attention_bind(*bound))
+        # bytes of split copies each call makes (0: it reads its rows as they are)
+        self._scratch = scratch
+        self._call = lib.hkv_segmented_attention_call_split if scratch else lib.hkv_segmented_attention_call
         self._out_shape = tuple(out_shape)
         self._out_dtype = out_dtype
         self._keep = keep  # tables, plan, offsets and workspace the bound pointers refer to
         self._dev = q.get_device()
         self._device = q.device
-        self._stream = a[-1]
+        self._stream = stream
         self._qs = q.shape
         self._ps = persisted_k.shape
         self._qdt, self._kdt, self._vdt = q.dtype, current_k.dtype, current_v.dtype
@@ -775,9 +770,20 @@ class BoundSegmentedAttention:
         stream = torch._C._cuda_getCurrentRawStream(dev)
         if stream != self._stream or torch.cuda.is_current_stream_capturing():
             return None
-        out = torch.empty(self._out_shape, dtype=self._out_dtype, device=self._device)
-        code = self._call(self._addr, q.data_ptr(), persisted_k.data_ptr(), persisted_v.data_ptr(),
-                          current_k.data_ptr(), current_v.data_ptr(), out.data_ptr(), stream)
+        tensors = (q.data_ptr(), persisted_k.data_ptr(), persisted_v.data_ptr(), current_k.data_ptr(),
+                   current_v.data_ptr())
+        if self._scratch:
+            if (tensors[1] | tensors[2] | tensors[3] | tensors[4]) & 15:
+                return None  # the operator copies rows that the split cannot read
+            try:
+                scratch = torch.empty(self._scratch, dtype=torch.uint8, device=self._device)
+            except torch.OutOfMemoryError:
+                return None  # ... and runs without the copies
+            out = torch.empty(self._out_shape, dtype=self._out_dtype, device=self._device)
+            code = self._call(self._addr, *tensors, out.data_ptr(), scratch.data_ptr(), self._scratch, stream)
+        else:
+            out = torch.empty(self._out_shape, dtype=self._out_dtype, device=self._device)
+            code = self._call(self._addr, *tensors, out.data_ptr(), stream)
         if code != 0:
             _lib.check(code)
         return out

@@ -282,6 +282,12 @@ int32_t hkv_segmented_attention_bind2(void* bound, int64_t bound_bytes, const in
                                       int64_t slab2_capacity, const int32_t* append2_offsets);
 int32_t hkv_segmented_attention_call(const void* bound, const void* q, void* slab_k, void* slab_v,
                                      const void* cur_k, const void* cur_v, void* out, void* stream);
+/* hkv_segmented_attention_split with a block bound by either call above
+ * (float32 q and k, default or tf32 dot modes): the float32 tensors and
+ * scratch 16-byte aligned, scratch as there. */
+int32_t hkv_segmented_attention_call_split(const void* bound, const void* q, void* slab_k, void* slab_v,
+                                           const void* cur_k, const void* cur_v, void* out, void* scratch,
+                                           int64_t scratch_bytes, void* stream);
 
 /*
  * Work plan of hkv_segmented_attention for host copies of its offset tables

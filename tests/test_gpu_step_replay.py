@@ -61,6 +61,36 @@ def test_replayed_generations_bit_identical(device, monkeypatch):
         assert np.array_equal(a, b), ("fused append off", t)
 
 
+def test_fp32_generations_are_replayed(device):
+    """All-fp32 steps, whose launches make split copies of K and V, are recorded
+    and repeated like the others: the same bits in later generations, also from
+    rows that start off a 16-byte boundary (which the operator takes)."""
+    sides = W.SIDES_1M[:9]
+    keep = W.sweep_keep_policies(layers=1, heads=16, sides=sides)[0]
+    cache = SegmentedLayerCache(W.schedule_from_keep(keep, sides), W.removed_from_keep(keep, len(sides)),
+                                num_heads=16)
+    inputs = [tuple(t.to(device).float() for t in x)
+              for x in W.generation_inputs(batch=2, heads=16, sides=sides, seed=2002)]
+    scale = 1.0 / math.sqrt(128)
+    first = _generation(cache, inputs, device, scale)
+    assert len(cache._replays) == len(sides)
+    assert all(r.attn._scratch > 0 for r in cache._replays.values())
+    for _ in range(2):
+        for t, (a, b) in enumerate(zip(first, _generation(cache, inputs, device, scale))):
+            assert np.array_equal(a, b), t
+    assert len(cache._replays) == len(sides)
+
+    def moved(t):
+        buf = torch.empty(t.numel() + 1, dtype=t.dtype, device=device)
+        buf[1:] = t.reshape(-1)
+        return buf[1:].view(t.shape)
+
+    off = [tuple(moved(t) for t in x) for x in inputs[-1:]]
+    for t, x in enumerate(inputs[:-1]):
+        cache.step(*x, t, scale)
+    assert np.array_equal(bits(cache.step(*off[0], len(sides) - 1, scale)), first[-1])
+
+
 def test_replay_keeps_slab_rows(device):
     """Every live slab row bit-exact after each replayed step (as the full
     steps leave it)."""
