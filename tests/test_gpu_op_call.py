@@ -120,8 +120,8 @@ def test_attention_taken(device, dtypes, kw, planned):
     (4, 16, 128, 8, True), (8, 32, 128, 8, False), (8, 33, 128, 8, True), (8, 32, 129, 8, True)])
 def test_fp32_split_copies_only_where_they_pay(device, B, H, L, cap, split, monkeypatch):
     """All-fp32 calls make split copies on the inner side of each limit and run
-    as they are, in no more memory than their outputs, on the other: both
-    paths of the operator alike."""
+    as they are, with no memory beside their outputs, on the other: both paths
+    of the operator alike."""
     g = torch.Generator(device=device).manual_seed(3)
     rand = lambda *s: torch.randn(s, generator=g, device=device)  # noqa: E731
     table = torch.zeros((H, 1), dtype=torch.int32, device=device)
@@ -143,8 +143,11 @@ def test_fp32_split_copies_only_where_they_pay(device, B, H, L, cap, split, monk
     staged, _ = measured(lambda: fused_real_pruning_flat_segmented_attention(**a))
     assert same(got, want) and same(got, staged) != split
     copies = 2 * 512 * B * (cap + H * L)
+    # torch's allocator leaves up to 1 MB of a cached block on one of over 1 MB, and rounds new ones up to 2 MB
+    rounding = 2 << 20
+    assert copies > 3 * rounding or split
     for n in (used, body_used):
-        assert (n >= copies) if split else (n < 4096)
+        assert (n >= copies) if split else (n < rounding)
 
 
 def test_fp32_call_without_room_for_split_copies(device, monkeypatch):
