@@ -26,7 +26,7 @@ HKV_ERR_DEVICE = -4
 
 # HKV_VERSION of include/heatkv.h these bindings follow (SIGNATURES below);
 # load() refuses a library built from another version of the header.
-ABI_VERSION = (0 << 16) | (3 << 8) | 0
+ABI_VERSION = (0 << 16) | (4 << 8) | 0
 
 DTYPE_CODES = {torch.float16: 1, torch.bfloat16: 2, torch.float32: 3}
 DTYPE_SPLIT_ROWS = 4  # K only: fp32 rows as bf16 high parts then low parts (hkv_split_rows)

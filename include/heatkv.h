@@ -50,7 +50,7 @@ int32_t hkv_concat_kv(const void* old_k, const void* new_k, const void* old_v, c
 /* Library version, (major << 16) | (minor << 8) | patch: HKV_VERSION of the
  * header the library was built with.  A loader compares it with the version
  * of the header (or bindings) it was written against and refuses a mismatch. */
-#define HKV_VERSION ((0 << 16) | (3 << 8) | 0)
+#define HKV_VERSION ((0 << 16) | (4 << 8) | 0)
 int32_t hkv_version(void);
 
 /* 1 when `device` is a gfx950 GPU this build can run on, else 0.

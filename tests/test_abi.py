@@ -46,7 +46,7 @@ def test_library_exports_every_declared_symbol():
 
 def test_version_and_host_only_calls():
     lib = _lib.load()
-    assert lib.hkv_version() == 0x000300 == _lib.ABI_VERSION
+    assert lib.hkv_version() == 0x000400 == _lib.ABI_VERSION
     assert lib.hkv_device_ok(-1) == 0
     assert isinstance(_lib.last_error(), str)
 
@@ -146,8 +146,8 @@ def test_bind_refuses_small_or_unbound_blocks():
     assert code == _lib.HKV_ERR_INVALID_ARG
 
 
-@pytest.mark.parametrize("source,missing", [("int hkv_version(void) { return 0x000300; }", "hkv_"),
-                                            ("int hkv_version(void) { return 0x000200; }", "ABI version 0.2.0"),
+@pytest.mark.parametrize("source,missing", [("int hkv_version(void) { return 0x000400; }", "hkv_"),
+                                            ("int hkv_version(void) { return 0x000300; }", "ABI version 0.3.0"),
                                             ("int hkv_something(void) { return 0; }", "ABI version 0.0.0")],
                          ids=["same version, fewer entry points", "other version", "no version"])
 def test_an_older_library_is_refused_with_the_way_out(source, missing, tmp_path, monkeypatch):
