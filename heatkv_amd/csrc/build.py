@@ -51,14 +51,21 @@ OP_CALL = os.path.join(PKG, "_op_call.so")
 
 def _op_call_command(out):
     """The extension's compile and link: torch's headers and libraries of the
-    running interpreter (already loaded when the package imports it)."""
+    running interpreter (already loaded when the package imports it).
+
+    NDEBUG keeps pybind11's thread-local reference counter out: after a library
+    with thread-local storage that a thread never touches is loaded, glibc
+    before 2.39 takes the slow path for every thread-local access of the others
+    (torch's among them): ``is_contiguous()`` 32 -> 44 ns, ``torch.empty`` 1.44 ->
+    1.77 us, a replayed step 7.5 -> 8.6 us."""
     import sysconfig
 
     import torch
 
     root = os.path.dirname(torch.__file__)
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
-    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    return ["g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-Wall",
+            "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
             f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-I{os.path.join(ROOT, 'include')}",
             "-isystem", os.path.join(root, "include"),
             "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"),

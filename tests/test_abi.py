@@ -201,3 +201,15 @@ def test_the_library_loads_without_the_extension(monkeypatch):
     with pytest.warns(RuntimeWarning, match="rebuild it with"):
         lib = _lib.load()
     assert lib.hkv_version() == _lib.ABI_VERSION and _lib.op_call is None
+
+
+def test_the_extension_has_no_thread_local_storage():
+    """A loaded library with thread-local storage that no thread touches slows
+    every torch call of the process (glibc before 2.39)."""
+    import struct
+
+    elf = open(os.path.join(os.path.dirname(_lib.LIB_PATH), "_op_call.so"), "rb").read()
+    phoff, = struct.unpack_from("<Q", elf, 32)
+    phentsize, phnum = struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, phoff + i * phentsize)[0] for i in range(phnum)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
