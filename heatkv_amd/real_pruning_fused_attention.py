@@ -770,20 +770,26 @@ class BoundSegmentedAttention:
         stream = torch._C._cuda_getCurrentRawStream(dev)
         if stream != self._stream or torch.cuda.is_current_stream_capturing():
             return None
-        tensors = (q.data_ptr(), persisted_k.data_ptr(), persisted_v.data_ptr(), current_k.data_ptr(),
-                   current_v.data_ptr())
         if self._scratch:
-            if (tensors[1] | tensors[2] | tensors[3] | tensors[4]) & 15:
-                return None  # the operator copies rows that the split cannot read
-            try:
-                scratch = torch.empty(self._scratch, dtype=torch.uint8, device=self._device)
-            except torch.OutOfMemoryError:
-                return None  # ... and runs without the copies
-            out = torch.empty(self._out_shape, dtype=self._out_dtype, device=self._device)
-            code = self._call(self._addr, *tensors, out.data_ptr(), scratch.data_ptr(), self._scratch, stream)
-        else:
-            out = torch.empty(self._out_shape, dtype=self._out_dtype, device=self._device)
-            code = self._call(self._addr, *tensors, out.data_ptr(), stream)
+            return self._launch_split(q, current_k, current_v, persisted_k, persisted_v, stream)
+        out = torch.empty(self._out_shape, dtype=self._out_dtype, device=self._device)
+        code = self._call(self._addr, q.data_ptr(), persisted_k.data_ptr(), persisted_v.data_ptr(),
+                          current_k.data_ptr(), current_v.data_ptr(), out.data_ptr(), stream)
+        if code != 0:
+            _lib.check(code)
+        return out
+
+    def _launch_split(self, q, current_k, current_v, persisted_k, persisted_v, stream):
+        """The launch of a split call: scratch for the copies beside the output."""
+        rows = (persisted_k.data_ptr(), persisted_v.data_ptr(), current_k.data_ptr(), current_v.data_ptr())
+        if (rows[0] | rows[1] | rows[2] | rows[3]) & 15:
+            return None  # the operator copies rows that the split cannot read
+        try:
+            scratch = torch.empty(self._scratch, dtype=torch.uint8, device=self._device)
+        except torch.OutOfMemoryError:
+            return None  # ... and runs without the copies
+        out = torch.empty(self._out_shape, dtype=self._out_dtype, device=self._device)
+        code = self._call(self._addr, q.data_ptr(), *rows, out.data_ptr(), scratch.data_ptr(), self._scratch, stream)
         if code != 0:
             _lib.check(code)
         return out
