@@ -539,7 +539,7 @@ __global__ __launch_bounds__(256, 2) void seg_attn_pipe_kernel(
 //    slots 8 g .. 8 g + 7 (g = l / 16) as keys 4 g .. + 3 and 16 + 4 g .. + 3,
 //    which is how S^T leaves the MFMA, and the V operand is read in that order.
 //  * A plan's 128-query units are run by two workgroups each, 8 ids apart (on
-//    one XCD).
+//    one XCD); by one up to 64 tokens.
 // us, seg_attn_pipe_kernel / here, B=2, 16 heads, a tenth retained: not planned
 // 4 tokens 7.8 / 6.8, 16: 7.9 / 6.9, 36: 8.5 / 7.4, 64: 9.4 / 8.1, 144: 11.2 / 9.9;
 // planned 6.5 / 6.1, 6.9 / 6.3, 7.1 / 6.6, 8.2 / 7.5, 10.2 / 9.7.  256 tokens,
@@ -577,13 +577,34 @@ inline int64_t items_of(const AttnArgs& a, int32_t queries) {
   return static_cast<int64_t>(a.batch) * a.heads * ((a.cur_len + queries - 1) / queries);
 }
 
-// Whether a launch runs seg_attn_small_kernel: few queries, a CU per 64-query
-// item, and items that seg_attn_pipe_kernel would not cut either -- a plan
-// without cut items (one unit per item), or no plan and a slab that holds few
-// rows per head (the rows that the tables retain are not known here; with
-// many, the parts of the round split are shorter than a whole item).
-inline bool small_launch(const AttnArgs& a, int64_t items, int32_t cus) {
-  if (a.cur_len > kSmallMaxLen || items_of(a, kSmallBM) > cus) return false;
+// Workgroups of such a launch: one per 64-query item, and two per plan unit
+// where a unit can hold two (uids and workgroup ids in eights), the second of
+// which leaves at once where it holds one.
+inline int64_t small_workgroups(const AttnArgs& a) {
+  if (a.plan == nullptr || a.cur_len <= kSmallBM) return items_of(a, kSmallBM);
+  return (items_of(a, 2 * kSmallBM) + 7) / 8 * 16;
+}
+
+// Whether a launch runs seg_attn_small_kernel: few queries, a CU per workgroup,
+// and items that seg_attn_pipe_kernel would not cut either -- a plan without
+// cut items (one unit per item), or no plan and a slab that holds few rows per
+// head (the rows that the tables retain are not known here; with many, the
+// parts of the round split are shorter than a whole item).  Its LDS leaves no
+// room for a second workgroup on a CU, so workgroups past the CUs wait for
+// whole items (planned, 80 items of 192 queries: 320 workgroups, 27.2 us against
+// 15.6), and the append's copy blocks run one at a time on the CUs that are left:
+// up to kSmallCopies writes of a block (one per destination) for each of those.
+// Dense steps with the append, us, seg_attn_pipe_kernel / here, by that number
+// (d: two destinations, u: not planned): 32 workgroups, 64 tokens 0.6: 10.0 / 9.5;
+// 192, 144 tokens 7: 14.7 / 13.9; 180, 36 tokens 7: 9.6 / 8.4, d 14: 10.0 / 9.3; 180,
+// 64 tokens 9.5: 11.1 / 10.8, u 11.2 / 10.1, d 19: 11.6 / 12.3; 192, 192 tokens u 12:
+// 12.8 / 11.9; 160, 128 tokens d 13: 13.8 / 13.3; 224, 36 tokens 21: 8.0 / 8.8, u 9.7 /
+// 10.2; 256, no CU left, 4 tokens 6.8 / 7.2, 64 tokens 12.1 / 15.0.
+constexpr int64_t kSmallCopies = 16;
+inline bool small_launch(const AttnArgs& a, int64_t items, int64_t copies, int32_t cus) {
+  if (a.cur_len > kSmallMaxLen || small_workgroups(a) > cus) return false;
+  if (a.append2_offsets != nullptr) copies *= 2;
+  if (copies > kSmallCopies * (cus - small_workgroups(a))) return false;
   return a.plan != nullptr ? a.plan_units == items
                            : a.slab_capacity <= static_cast<int64_t>(kSmallRowsPerHead) * a.heads;
 }
@@ -617,7 +638,7 @@ __global__ __launch_bounds__(256, 1) void seg_attn_small_kernel(const int32_t* _
   const bool planned = plan_p != nullptr;
   if (planned) {
     const int32_t id = static_cast<int32_t>(blockIdx.x);
-    const int32_t uid = ((id >> 4) << 3) + (id & 7);
+    const int32_t uid = n_qt > 1 ? ((id >> 4) << 3) + (id & 7) : id;
     if (uid >= n_units) return;
     const int32_t* pu = plan_p + static_cast<int64_t>(uid) * kPlanInts;
     const int32_t ph = pu[0], pj = pu[1];
@@ -625,7 +646,7 @@ __global__ __launch_bounds__(256, 1) void seg_attn_small_kernel(const int32_t* _
     if (ph < 0 || ph >= H || pj < 0 || pj >= a.batch * n_qt2) return;  // not a unit of this launch
     w.h = ph;
     w.b = pj / n_qt2;
-    w.qt = 2 * (pj - w.b * n_qt2) + ((id >> 3) & 1);
+    w.qt = n_qt > 1 ? 2 * (pj - w.b * n_qt2) + ((id >> 3) & 1) : 0;
     if (w.qt >= n_qt) return;
     w.bh = w.b * H + w.h;
   } else {
@@ -904,8 +925,8 @@ hipError_t launch(const AttnArgs& a, const Scalars& s, hipStream_t st) {
   const int64_t blocks = a.plan != nullptr ? (a.plan_units > 0 ? a.plan_units : 0) : split_units(split);
   if (blocks + copies <= 0) return hipSuccess;
   if (blocks + copies > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-  if (small_launch(a, items, cus)) {
-    const int64_t small = a.plan != nullptr ? (blocks + 7) / 8 * 16 : items_of(a, kSmallBM);
+  if (small_launch(a, items, copies, cus)) {
+    const int64_t small = small_workgroups(a);
     if (small + copies > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     b.append_first = static_cast<int32_t>(small);
     seg_attn_small_kernel<DT, VDT><<<dim3(static_cast<uint32_t>(small + copies)), 256, 0, st>>>(
