@@ -543,8 +543,8 @@ __device__ __forceinline__ uint32_t pack2_rest(float x, float y, uint32_t hi) {
 // MIXED: tile nfull holds the current rows' last `rest` and the first prior
 // rows, as in the 16-bit kernel (seg_attn_pipe_kernel, where the lines of the
 // rule are drawn): its DMAs are issued for the lanes of current rows and again
-// for the lanes of prior rows.  With or without it, a last half without keys is
-// left out.
+// for the lanes of prior rows.  A last half without keys is left out (kOdd; not
+// with 16-bit V beyond the mixed lengths, where its masked half runs).
 template <int VDT, bool MIXED>
 __global__ __launch_bounds__(kHThreads, 2) void seg_attn_half_kernel(const int32_t* __restrict__ plan_p,
                                                                     const int32_t n_units, const AttnArgs a,
@@ -935,29 +935,41 @@ hipError_t launch_half(const AttnArgs& a, const Scalars& s, hipStream_t st, int3
 // Whether a call on split K rows with 16-bit V runs as 128-query workgroups
 // (seg_attn_half_kernel; a plan's 256-query units as two halves each) instead
 // of 256-query ones.  The 8-wave form is the faster one once every CU has its
-// fill of it (546 against 592 us on the 2B final step, 512 items of 256
-// queries; 198 / 204 at 288 items), the halves before that: they spread over
-// twice the workgroups, a last tile of at most 128 queries costs half, and a
-// call without a plan cuts its items in two (one image pair, 16 heads, us,
-// halves / 8 waves at 144, 400, 576, 1024, 1600, 2304 tokens: planned 16.1 /
-// 19.5, 25.7 / 33.0, 30.7 / 39.9, 59.2 / 63.6, 105.0 / 107.1, 204 / 198; not
-// planned 17.2 / 20.4, 26.9 / 33.8, 37.0 / 47.2, 58.5 / 96.9, 105.7 / 126,
-// 203 / 229; not planned 4096 tokens 613 / 587).  So, with a plan: up to one
-// 128-query workgroup per CU, and up to one 256-query item per CU from 2048
-// tokens (between the two some CUs share two halves while others have one:
-// 1024 tokens, B=3, 12 heads 61.6 / 59.4; 1008 tokens, 16 heads, a twentieth
-// retained 65.8 / 59.2; 1600 tokens, uneven heads 109.8 / 108.6; but 2304 tokens,
-// B=1 111.8 / 117.0); without one: below two 256-query items per CU.  And where
-// half tiles save at least an eighth of the padded queries (576 tokens, 768
-// items: 135 / 143 us; 1600 tokens save 7 %: 771 / 753).
+// fill of it, the halves before that: they spread over twice the workgroups, a
+// last tile of at most 128 queries costs half, a call without a plan cuts its
+// items in two (one image pair, 16 heads, not planned, us, halves / 8 waves at
+// 144, 576, 1024, 1600, 2304, 4096 tokens: 17.2 / 20.4, 37.0 / 47.2, 58.5 / 96.9,
+// 105.7 / 126, 203 / 229, 613 / 587), and their launch takes the append, which
+// follows the 8-wave one as a launch of its own.  16 heads, a tenth retained /
+// heads of uneven lengths, planned, K split by the producer, us, halves : 8 waves
+// by 256-query items:
+// * no append, up to one half per CU: 64 items (1024 tokens) 34.8 : 43.6 / 42.8 :
+//   56.6, 112 (1600) 63.7 : 62.0 / 74.9 : 80.9, 128 (B=2, 1024) 50.8 : 52.2 / 62.1 :
+//   63.8.  Above, some CUs share two halves while others have one: 144 (2304)
+//   115.9 : 105.2 / 129 : 133, 192 (B=2, 1296) 90.9 : 82.9 / 100.4 : 98.0, 224 (B=2,
+//   1600) 109.7 : 101.7 / 127.2 : 130.3, 256 (4096) 283 : 259 / 331 : 317.
+// * with the append, up to two items per CU (where every head appends) and
+//   2560 tokens: 192 (B=2, 1296) 92.1 : 92.7 / 101.7 : 109.1, 192 (B=3, 1024)
+//   77.0 : 81.1 / 90.6 : 97.3, 224 111.5 : 115.2 / 130 : 144, 288 (B=2, 2304) 218 : 222 /
+//   235 : 239, 432 (B=3, 2304) 314 : 318 / 352 : 351, but 176 (2704) 169 : 155 / 174 :
+//   180, 256 (4096) 286 : 275 / 333 : 332, and 660 (B=2, 30 heads, 2704) 522 : 513.
+// Without a plan: below two 256-query items per CU.  And where half tiles save
+// at least an eighth of the padded queries (576 tokens, 768 items: 135 / 143 us;
+// 1600 tokens save 7 %: 771 / 753).
+constexpr int32_t kHalvesAppendLen = 2560;
 bool split_in_halves(const AttnArgs& a) {
   int device = 0;
-  const int32_t cus = hipGetDevice(&device) == hipSuccess ? split_slots(device) / 2 : 0;
+  const int64_t cus = hipGetDevice(&device) == hipSuccess ? split_slots(device) / 2 : 0;
   const int64_t t256 = (static_cast<int64_t>(a.cur_len) + kSBM - 1) / kSBM;
   const int64_t t128 = (static_cast<int64_t>(a.cur_len) + 127) / 128;
   const int64_t items = static_cast<int64_t>(a.batch) * a.heads * t256;
-  const int64_t few = a.cur_len >= 2048 ? items : 2 * items;
-  if (a.plan != nullptr ? few <= cus : items < 2 * static_cast<int64_t>(cus)) return true;
+  if (a.plan == nullptr) {
+    if (items < 2 * cus) return true;
+  } else if (a.append_offsets != nullptr && a.cur_len <= kHalvesAppendLen) {
+    if (items <= 2 * cus) return true;
+  } else if (2 * items <= cus) {
+    return true;
+  }
   return 8 * t128 <= 7 * 2 * t256;
 }
 

@@ -81,3 +81,12 @@ def check_append(device, B, H, L, qk, kept, dests, plans):
                                          (2, 5, 65, 2), (1, 3, 192, 2), (1, 2, 193, 1)])
 def test_small_launches_with_the_append(B, H, L, dests, device):
     check_append(device, B, H, L, torch.bfloat16, lambda h: (h * 13) % 40, dests, {"planned": 1, "unplanned": None})
+
+
+# 128-query form (plan units of 256 queries as two workgroups, the last one empty
+# at L % 256 in 1 .. 128), then past its two lines: 2560 tokens, two items a CU
+@pytest.mark.parametrize("B,H,L", [(2, 3, 100), (2, 3, 300), (1, 5, 129), (2, 2, 1000), (1, 13, 2700), (4, 131, 250)])
+@pytest.mark.parametrize("dests", [1, 2])
+def test_split_row_launches_with_the_append(B, H, L, dests, device):
+    plans = {"planned": 1, "cut": 4, "unplanned": None} if H < 10 else {"planned": 1}
+    check_append(device, B, H, L, torch.float32, lambda h: (h * 97) % 700 if H < 100 else h % 7, dests, plans)
