@@ -19,7 +19,8 @@
 // now (6.3 TB/s; non-temporal loads or stores alone 102, neither 106).  B=2, 16
 // items: 2304 rows 12.5 / 12.4 us, 576 rows 4.6 / 3.8, 64 rows 3.4 / 2.4.
 // Workgroups whose chunk lies beyond their item's length exit at once (append
-// items all share one length, so none are idle there).
+// items all share one length, so none are idle there), ~0.4 ns each: lists of
+// very uneven lengths, where most do, take 64-row chunks (kUneven).
 #include "hkv_internal.h"
 #include "stream_mem.h"
 
@@ -28,8 +29,18 @@ namespace {
 
 constexpr int kThreads = 256;
 constexpr int kChunkRows = 16;
-constexpr int kChunkRowsWide = 64;  // where 16-row chunks would be more workgroups than a launch takes
 constexpr int64_t kMaxBlocks = 0xffffffffLL / kThreads;  // a launch has fewer than 2^32 threads in x
+// 64-row chunks, K before V, four vectors of one tensor in flight per thread and
+// ordinary accesses: where 16-row chunks would be more workgroups than a launch
+// takes, and where the longest item times the items is over kUneven times the
+// rows that can move (all rows of the smaller tensor).  bf16, one item of 2304
+// rows among shorter ones for each of 16 heads, B=2, us, 16-row / 64-row chunks,
+// the same tensors again / tensors from HBM, by that ratio: 3.2 50.3 : 49.8 / 52.6 :
+// 58.7, 5.4 30.0 : 26.4 / 30.9 : 32.8, 7.1 29.3 : 22.4 / 29.8 : 27.5, 11 28.2 : 16.1 /
+// 28.3 : 21.0, 43 110 : 32 / 110 : 34; B=8, 32 heads 3.2 395 : 473 / 404 : 472, 5.4 213 :
+// 241 / 219 : 233, 7.1 208 : 200 / 213 : 196, 43 858 : 245 / 861 : 246.
+constexpr int kChunkRowsWide = 64;
+constexpr int64_t kUneven = 6;
 constexpr int kUnroll = 4;
 
 typedef uint32_t U16B __attribute__((ext_vector_type(4)));
@@ -104,10 +115,17 @@ __global__ __launch_bounds__(kThreads) void pack_kernel(PackArgs a, int32_t chun
   const int64_t D = a.head_dim;
   const int64_t src_elem = b * a.src_batch_stride + (s0 + lo) * D;
   const int64_t dst_elem = b * a.dst_batch_stride + (d0 + lo) * D;
-  copy_ranges<UK, UV>(static_cast<char*>(a.dst_k) + dst_elem * a.k_elem_bytes,
-                      static_cast<const char*>(a.src_k) + src_elem * a.k_elem_bytes, rows * D * a.k_elem_bytes,
-                      static_cast<char*>(a.dst_v) + dst_elem * a.v_elem_bytes,
-                      static_cast<const char*>(a.src_v) + src_elem * a.v_elem_bytes, rows * D * a.v_elem_bytes);
+  char* const dk = static_cast<char*>(a.dst_k) + dst_elem * a.k_elem_bytes;
+  char* const dv = static_cast<char*>(a.dst_v) + dst_elem * a.v_elem_bytes;
+  const char* const sk = static_cast<const char*>(a.src_k) + src_elem * a.k_elem_bytes;
+  const char* const sv = static_cast<const char*>(a.src_v) + src_elem * a.v_elem_bytes;
+  const int64_t k_bytes = rows * D * a.k_elem_bytes, v_bytes = rows * D * a.v_elem_bytes;
+  if (chunk_rows == kChunkRows) {
+    copy_ranges<UK, UV>(dk, sk, k_bytes, dv, sv, v_bytes);
+  } else {
+    copy_range<UK>(dk, sk, k_bytes);
+    copy_range<UV>(dv, sv, v_bytes);
+  }
 }
 
 // Widest copy unit (16, 4 or 2 bytes) that keeps every access aligned.
@@ -180,7 +198,9 @@ hipError_t launch_pack(const PackArgs& a, hipStream_t stream) {
   if (a.n_items <= 0 || a.row_limit <= 0 || a.batch <= 0) return hipSuccess;
   int32_t chunk_rows = kChunkRows;
   auto count = [&] { return (static_cast<int64_t>(a.row_limit) + chunk_rows - 1) / chunk_rows; };
-  if (count() * a.n_items > kMaxBlocks) chunk_rows = kChunkRowsWide;
+  const int64_t rows = a.src_rows < a.dst_rows ? a.src_rows : a.dst_rows;
+  if (count() * a.n_items > kMaxBlocks || static_cast<int64_t>(a.n_items) * a.row_limit / kUneven > rows)
+    chunk_rows = kChunkRowsWide;
   const int64_t chunks64 = count();
   const int64_t blocks = chunks64 * a.n_items;
   if (blocks > 0x7fffffffLL) return hipErrorInvalidConfiguration;

@@ -13,10 +13,13 @@ from support import bits
 pytestmark = pytest.mark.gpu
 
 
+# Among them: a list uneven enough for 64-row chunks (33 items x 700 rows against
+# 1388 that move) and one that is not (33 x 130 against 930).
 # The last two: so many items that 16-row chunks would pass the launch grid
 # (64-row chunks run: 66000 x 256 chunks of 16 rows), and 2-byte units.
 @pytest.mark.parametrize("lengths,D,max_length", [
     ([1, 15, 16, 17, 31, 32, 33, 64, 65], 128, 65), ([2], 128, 2), ([47, 0, 48], 128, 48),
+    ([700] + [1, 3, 17, 65] * 8, 128, 700), ([130] + [1, 3, 31, 65] * 8, 128, 130),
     ([5, 70, 16, 64, 4000, 65] + [0] * 66000 + [17, 130], 6, 4096), ([17, 16, 3], 5, 17)])
 @pytest.mark.parametrize("kdt,vdt", [(torch.bfloat16, torch.bfloat16), (torch.float32, torch.bfloat16)])
 def test_pack_chunk_edges(lengths, D, max_length, kdt, vdt, device):
