@@ -163,14 +163,23 @@ def test_fp32_call_without_room_for_split_copies(device, monkeypatch):
     assert not same(fn(**a), want)  # split where there is room
     torch.cuda.synchronize(device)
     torch.cuda.empty_cache()
-    room = torch.cuda.memory_reserved(device) + (24 << 20)  # the output fits, 64 MB of copies do not
+    room = torch.cuda.memory_reserved(device) + (24 << 20)
+    held = []
     try:
         torch.cuda.set_per_process_memory_fraction(room / torch.cuda.get_device_properties(device).total_memory, device)
+        # fill what earlier tests left in the allocator's segments, then leave one hole: it and
+        # the free rest beside it take the output, not 64 MB of copies
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:
+                held.append(torch.empty(8 << 20, dtype=torch.uint8, device=device))
+        held.pop()
         for call in (fn, lambda **kw: body(fn, **kw)):
             got = call(**a)
             torch.cuda.synchronize(device)
             assert same(got, want)
+            del got
     finally:
+        held.clear()
         torch.cuda.set_per_process_memory_fraction(1.0, device)
 
 
