@@ -2,11 +2,11 @@
 // (attention, the QKV producer, the slab pack): the Python extension
 // heatkv_amd._op_call.
 //
-// A small launch runs 8-9 us on the device, but checking eight tensors, reading
+// A small launch runs 6-8 us on the device, but checking eight tensors, reading
 // the knobs and marshalling about thirty arguments cost the Python operator
 // 15-16 us per call, so calls on early scales ran at the host's pace.  Here the
 // same checks read the tensors in C++ (nothing is remembered from one call for
-// the next), the outputs are allocated and the library is called: 16.7 -> 7.7 us
+// the next), the outputs are allocated and the library is called: 16.4 -> 6.1 us
 // per call of 16 tokens (B=2, 16 heads), back to back; a whole layer's ten small
 // scales at B=1 966 -> 837 us.
 //

@@ -40,7 +40,14 @@ int32_t attention_workgroups_per_cu(const AttnArgs& a) {
   if (a.k_dtype == kSplitRows) return 1;
   if (!force_staged() && attention_direct_supported(a)) return 2;
   // the staged kernel's split modes (3-piece q/k, fp32 value mode, fp32 V)
-  // hold more pieces per wave: one workgroup per CU
+  // hold more pieces per wave: one workgroup per CU.  All-fp32 calls at the
+  // default modes mostly run seg_attn_half_kernel, two per CU, but are planned
+  // for one too: a plan's part and unit costs are the 16-bit kernel's, and with
+  // 512 slots the plan search leaves whole items where cuts pay (whole calls,
+  // 16 heads, a tenth retained / uneven heads, us, planned for 256 / 512 slots:
+  // 1296 tokens, B=2 132.5 : 150 / 157 : 168, 1600 175 : 184 / 209 : 213, 400, B=4
+  // 51.7 : 51.5 / 62 : 70; but 1600, B=1 104.5 : 103 / 132 : 117, 2304, B=4 636 : 613 /
+  // 726 : 704).
   const bool split = (a.q_dtype == kF32 && a.qk_dot_mode == kDotFp32) || a.value_dot_mode == kDotFp32 ||
                      a.v_dtype == kF32;
   return split ? 1 : 2;

@@ -230,10 +230,13 @@ def attention_item_shape(q_dtype, k_dtype, v_dtype, *, k_split_rows: bool = Fals
     None), as the library reports them (``hkv_segmented_attention_item_shape``):
     the ``queries_per_item`` and ``slots`` of :func:`segmented_attention_plan`.
     Items are 128 queries, or 256 for the 8-wave form of the split-row
-    kernel; slots are the resident workgroups of that kernel (2 per CU for
-    the 16-bit kernel and the staged kernel's plain modes, 1 per CU for the
-    split-row kernel and the staged kernel's split modes).  slots is None
-    for a device that is not a GPU (no kernel runs there)."""
+    kernel; slots are the workgroups a plan is best made for: the resident
+    ones (2 per CU for the 16-bit kernel and the staged kernel's plain modes,
+    1 per CU for the split-row kernel and the staged kernel's split modes),
+    except that all-fp32 calls keep the staged kernel's 1 per CU where the
+    128-query split-row kernel runs 2 (the library has the figures beside the
+    rule).  slots is None for a device that is not a GPU (no kernel runs
+    there)."""
     dev = torch.device("cuda") if device is None else torch.device(device)
     if dev.type != "cuda":
         return (attention_queries_per_item(q_dtype, k_dtype, v_dtype, k_split_rows=k_split_rows), None)

@@ -326,8 +326,10 @@ int32_t hkv_segmented_attention_plan(const int32_t* seg_starts, const int32_t* s
  * writes the device's resident attention workgroups for the kernel that runs
  * (2 per CU for the 16-bit kernel and the staged kernel's plain modes, 1 per
  * CU for split K rows and for the staged kernel's fp32 QK dot mode on fp32 q,
- * fp32 value dot mode and fp32 V) to *slots when slots is not NULL (the
- * `queries_per_item` and `slots` of hkv_segmented_attention_plan); a negative
+ * fp32 value dot mode and fp32 V -- also for the split call on fp32 V, whose
+ * kernel runs 2, as plans for 1 are the better ones on the whole) to *slots
+ * when slots is not NULL (the `queries_per_item` and `slots` of
+ * hkv_segmented_attention_plan); a negative
  * HKV_ERR_* code when the device cannot be queried.  No counterpart in the
  * reference.
  */
